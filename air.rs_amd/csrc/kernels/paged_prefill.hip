@@ -60,6 +60,7 @@
 #include "../pool.hpp"
 #include "codecs.hpp"
 #include "prefill_common.hpp"
+#include "prefill_rank.hpp"
 
 namespace airkv {
 namespace {
@@ -271,40 +272,11 @@ __device__ __forceinline__ void to_bf16x8_split(const Raw8<DT> &r, u32x4 &hi, u3
 // gets exactly one rank whatever the lengths hold.  Batches above kRankCap
 // sequences or kRankItems items are taken slot by slot (slot slowest),
 // without ranking or splitting.
-constexpr int kRankCap = 2048;
-constexpr int kRankItems = 64 * kThreads;
-constexpr int kRankLdsBytes = (kThreads + kWaves + 8 + 2 * kRankCap) * 4;
 
 struct PrefillSlot {
     int b, kh, z, nz;
     int p, ns, ord;            // piece, pieces of the slot (1: not split), split ordinal (-1: none)
 };
-
-__device__ __forceinline__ int len_bucket(int64_t len) {   // 0 .. 248, monotone in len
-    if (len <= 0) return 0;
-    const uint32_t x = len > 0x7fffffff ? 0x7fffffffu : (uint32_t)len;
-    const int e = 31 - __builtin_clz(x);
-    const int m = e >= 3 ? (int)(x >> (e - 3)) & 7 : (int)(x << (3 - e)) & 7;
-    return 1 + 8 * e + m;
-}
-
-// Exclusive prefix sum over the workgroup's threads in thread order; wsum
-// holds kWaves ints of LDS.  Contains barriers: every thread calls it.
-__device__ __forceinline__ int block_exclusive_scan(int v, int *wsum) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int incl = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(incl, o);
-        if (lane >= o) incl += y;
-    }
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    int base = 0;
-    for (int w = 0; w < wave; ++w) base += wsum[w];
-    __syncthreads();
-    return base + incl - v;
-}
 
 // Keys the heaviest wave of slot z of a sequence needs (0: no work).
 __device__ __forceinline__ int64_t slot_keys(int64_t len, int64_t qlen, int G, int z) {
@@ -330,21 +302,6 @@ __device__ __forceinline__ int slot_pieces(int64_t tiles, int64_t T, int ns_max)
     return (int)(n < ns_max ? n : ns_max);
 }
 
-// Whether sequence b's rows and length are consistent: 0 <= cu_q[b] <=
-// cu_q[b + 1] <= total_q, 0 <= seq_len <= max_blocks * block_size and
-// q_len <= seq_len.  The one test every prefill kernel applies: an
-// inconsistent sequence is counted and zero-filled by its first workgroup,
-// never split into pieces and never written by the merge.
-__device__ __forceinline__ bool prefill_rows_ok(const PrefillArgs &a, int b) {
-    const int32_t q0 = a.cu_q[b], q1 = a.cu_q[b + 1];
-    return q0 >= 0 && q1 >= q0 && q1 <= a.total_q;
-}
-__device__ __forceinline__ bool prefill_seq_ok(const PrefillArgs &a, int b) {
-    const int64_t len = a.lens[b];
-    const int64_t qlen = (int64_t)a.cu_q[b + 1] - a.cu_q[b];
-    return prefill_rows_ok(a, b) && len >= 0 && len <= a.max_len && qlen <= len;
-}
-
 // The plan of a split launch: one int2 per grid row {item, slot info}.
 __device__ __forceinline__ int2 *prefill_plan_table(const PrefillArgs &a) {
     return reinterpret_cast<int2 *>((uint8_t *)a.ws + 64 + 16 * (int64_t)a.ws_units);
@@ -355,7 +312,6 @@ __device__ __forceinline__ int2 *prefill_plan_table(const PrefillArgs &a) {
 // workgroup.  lds: at least kThreads + kWaves + 8 + 2 * kRankCap ints, free
 // for the duration.
 __device__ PrefillSlot prefill_slot(const PrefillArgs &a, int *lds) {
-    const int tid = threadIdx.x;
     const int nz = a.nz, nsm = a.ns_max;
     const int row = (int)(blockIdx.x / (unsigned)a.n_kv_heads);
     PrefillSlot sl;
@@ -381,48 +337,10 @@ __device__ PrefillSlot prefill_slot(const PrefillArgs &a, int *lds) {
         sl.z = row / a.batch;
         return sl;
     }
-    int *hist = lds, *wsum = lds + kThreads, *sel = lds + kThreads + kWaves;
-    int *slen = sel + 8, *sq = slen + kRankCap;
-    hist[tid] = 0;
-    for (int i = tid; i < a.batch; i += kThreads) {
-        slen[i] = a.lens[i];
-        const int64_t ql = (int64_t)a.cu_q[i + 1] - a.cu_q[i];
-        sq[i] = ql < 0 ? 0 : ql > 0x7fffffff ? 0x7fffffff : (int)ql;
-    }
-    __syncthreads();
-    const int n_it = a.batch * nz;
-    const int chunk = (n_it + kThreads - 1) / kThreads;
-    const int i0 = tid * chunk, i1 = i0 + chunk < n_it ? i0 + chunk : n_it;
-    auto bucket_of = [&](int i) {
-        const int bb = i / nz;
-        return len_bucket(slot_keys(slen[bb], sq[bb], a.group, i - bb * nz));
-    };
-    for (int i = i0; i < i1; ++i) atomicAdd(&hist[bucket_of(i)], 1);
-    __syncthreads();
-    // buckets in decreasing order: thread t takes bucket kThreads - 1 - t
-    const int bucket = kThreads - 1 - tid;
-    const int cnt = hist[bucket];
-    const int start = block_exclusive_scan(cnt, wsum);
-    if (row >= start && row < start + cnt) {
-        sel[0] = bucket;
-        sel[1] = row - start;
-    }
-    __syncthreads();
-    const int want = sel[0], j = sel[1];
-    // the j-th item (index order) of bucket want: thread t scans its chunk
-    int c = 0;
-    for (int i = i0; i < i1; ++i) c += bucket_of(i) == want;
-    const int before = block_exclusive_scan(c, wsum);
-    if (j >= before && j < before + c) {
-        int k = j - before;
-        for (int i = i0; i < i1; ++i)
-            if (bucket_of(i) == want && k-- == 0) sel[0] = i;
-    }
-    __syncthreads();
-    const int item = sel[0];
+    const int item = rank_item(a, lds, nz, row,
+                               [&](int64_t len, int64_t qlen, int z) { return slot_keys(len, qlen, a.group, z); });
     sl.b = item / nz;
     sl.z = item - sl.b * nz;
-    __syncthreads();   // the caller reuses the LDS
     return sl;
 }
 
@@ -543,47 +461,6 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PrefillArgs 
         const int r = atomicAdd(&cnt[bucket_of(i)], 1);
         plan[r] = int2{i, info[i / nsm]};
     }
-}
-
-// Per-(sequence, kv head) setup shared by the prefill kernels: reads the
-// sequence's rows and length, counts (once) an inconsistent sequence and
-// every out-of-pool table entry within its length, zero-fills the rows of an
-// inconsistent sequence, and returns whether the workgroup has rows to
-// compute.  Uniform per workgroup.
-template <int BS>
-__device__ bool prefill_begin(const PrefillArgs &a, const PrefillSlot &sl, int32_t &q0, int &qlen, int64_t &len) {
-    const int b = sl.b, kh = sl.kh, tid = threadIdx.x;
-    const int G = a.group;
-    q0 = a.cu_q[b];
-    len = a.lens[b];
-    qlen = a.cu_q[b + 1] - q0;
-    const bool rows_ok = prefill_rows_ok(a, b);
-    const bool seq_ok = prefill_seq_ok(a, b);
-    const int32_t *tbl = a.tables + (int64_t)b * a.max_blocks;
-    if (sl.z == 0 && sl.p == 0 && kh == 0) {
-        if (!seq_ok) {
-            if (tid == 0) atomicAdd(a.errors, 1ull);
-        } else if (qlen > 0) {
-            for (int64_t j = tid; j < (len + BS - 1) / BS; j += kThreads) {
-                const int32_t blk = tbl[j];
-                if (blk < 0 || blk >= a.num_blocks) atomicAdd(a.errors, 1ull);
-            }
-        }
-    }
-    if (!seq_ok) {
-        // rows of a sequence whose lengths are inconsistent become zeros
-        if (rows_ok && sl.z == 0 && sl.p == 0) {
-            const int64_t n = (int64_t)qlen * G * D;
-            for (int64_t i = tid; i < n; i += kThreads) {
-                const int64_t r = i / (G * D), e = i % (G * D);
-                const int64_t idx = ((int64_t)(q0 + r) * a.n_q_heads + kh * G) * D + e;
-                if (a.out_dtype == AIR_KV_F32) ((float *)a.out)[idx] = 0.0f;
-                else ((uint16_t *)a.out)[idx] = 0;
-            }
-        }
-        return false;
-    }
-    return qlen > 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -809,7 +686,8 @@ void prefill_pipe_kernel(PrefillArgs a) {
     int32_t q0;
     int qlen;
     int64_t len;
-    if (!prefill_begin<BS>(a, sl, q0, qlen, len)) return;
+    if (!prefill_begin(a, b, kh, sl.z == 0 && sl.p == 0, D, q0, qlen, len)) return;
+    if (sl.z == 0 && sl.p == 0 && kh == 0) prefill_count_entries(a, b, BS, len);
     const int32_t *tbl = a.tables + (int64_t)b * a.max_blocks;
     const int q_offset = (int)(len - qlen);
     const int ntb = (qlen + kRows - 1) / kRows;

@@ -14,7 +14,7 @@ struct PrefillArgs {
     int32_t batch, max_blocks, total_q;
     int64_t max_len;               // max_blocks * block_size (set by launch_prefill)
     float scale_log2;              // softmax scale * log2(e)
-    int32_t n_kv_heads, group, scale_group;
+    int32_t n_kv_heads, group, scale_group, head_dim, block_size;
     int64_t num_blocks;
     const void *k_pages, *v_pages;
     const float *k_scales, *v_scales;
@@ -27,6 +27,7 @@ struct PrefillArgs {
     int32_t slots;                 // resident workgroups of the launch: the balance target
     void *ws;                      // key-split workspace (ns_max > 1)
     int32_t ws_units;              // split slots the workspace holds
+    bool fp8;                      // launch_prefill_f32: 1-byte pages hold fp8 codes (else int8)
 };
 
 // Key-split workspace: a 64-byte header (int32 count of split slots), one
@@ -50,5 +51,9 @@ bool prefill_supported(int dtype, int head_dim, int block_size, int scale_group)
 // a.ws / a.ws_units: the workspace, or NULL / 0 for no key split
 hipError_t launch_prefill(PrefillArgs a, int dtype, int block_size, int32_t max_q_len, int cus,
                           hipStream_t s);
+// Prefill at f32 precision, for every pool prefill_supported refuses.
+hipError_t launch_prefill_f32(PrefillArgs a, int dtype, int32_t max_q_len, int cus, hipStream_t s);
+// Whether it beats launch_prefill_rows for this launch.
+bool prefill_f32_better(const PrefillArgs &a, int dtype, int32_t max_q_len);
 
 }  // namespace airkv

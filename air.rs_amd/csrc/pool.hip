@@ -209,7 +209,7 @@ int air_paged_prefill_workspace_size(const air_kv_pool *p, int32_t n_q_heads, in
     if (batch < 0 || max_q_len < 0) return fail(AIR_KV_E_INVALID_ARG, "negative batch or max_q_len");
     const air_kv_pool_desc &d = p->desc;
     if (batch == 0 || !airkv::prefill_supported(d.dtype, d.head_dim, d.block_size, d.scale_group)) {
-        *bytes = 0;             // the vector prefill splits nothing
+        *bytes = 0;             // these pools' prefills use no workspace
         return AIR_KV_OK;
     }
     const airkv::PrefillPlan pl =
@@ -241,27 +241,30 @@ int air_paged_prefill(air_kv_pool *p, void *stream, const void *q, int32_t q_dty
         return fail(AIR_KV_E_INVALID_ARG, "prefill scale must be finite and > 0");
     if ((int64_t)max_blocks * d.block_size > INT32_MAX)
         return fail(AIR_KV_E_INVALID_ARG, "max_blocks * block_size exceeds int32");
-    if (!airkv::prefill_supported(d.dtype, d.head_dim, d.block_size, d.scale_group)) {
-        // F32 pages, head_dim other than 128, small scale groups: the
-        // vector kernel, one query row per workgroup and head chunk
-        if (batch > 65535) return fail(AIR_KV_E_INVALID_ARG, "batch %d above 65535 for this pool", batch);
-        hipError_t e = airkv::launch_prefill_rows(*p, (hipStream_t)stream, q, q_dtype, n_q_heads, cu_q, total_q,
-                                                  max_q_len, block_tables, seq_lens, batch, max_blocks, scale,
-                                                  out, out_dtype);
-        return e == hipSuccess ? AIR_KV_OK : hip_fail(e, "air_paged_prefill launch");
-    }
     airkv::PrefillArgs a;
     a.q = q; a.q_dtype = q_dtype; a.n_q_heads = n_q_heads;
     a.cu_q = cu_q; a.tables = block_tables; a.lens = seq_lens;
     a.batch = batch; a.max_blocks = max_blocks; a.total_q = total_q;
     a.scale_log2 = scale * 1.4426950408889634f;
     a.n_kv_heads = d.n_kv_heads; a.group = n_q_heads / d.n_kv_heads; a.scale_group = d.scale_group;
+    a.head_dim = d.head_dim; a.block_size = d.block_size;
     a.num_blocks = d.num_blocks;
     a.k_pages = p->k_pages; a.v_pages = p->v_pages; a.k_scales = p->k_scales; a.v_scales = p->v_scales;
     a.out = out; a.out_dtype = out_dtype;
     a.errors = p->errors;
     a.ws = nullptr;
     a.ws_units = 0;
+    if (!airkv::prefill_supported(d.dtype, d.head_dim, d.block_size, d.scale_group)) {
+        // F32 pages, head_dim other than 128: the f32-precision kernel, or
+        // for launches too small for it the vector kernel
+        if (batch > 65535) return fail(AIR_KV_E_INVALID_ARG, "batch %d above 65535 for this pool", batch);
+        hipError_t e = airkv::prefill_f32_better(a, d.dtype, max_q_len)
+                           ? airkv::launch_prefill_f32(a, d.dtype, max_q_len, p->cus, (hipStream_t)stream)
+                           : airkv::launch_prefill_rows(*p, (hipStream_t)stream, q, q_dtype, n_q_heads, cu_q, total_q,
+                                                        max_q_len, block_tables, seq_lens, batch, max_blocks, scale,
+                                                        out, out_dtype);
+        return e == hipSuccess ? AIR_KV_OK : hip_fail(e, "air_paged_prefill launch");
+    }
     const airkv::PrefillPlan pl =
         airkv::prefill_plan(batch, d.n_kv_heads, n_q_heads / d.n_kv_heads, max_q_len, p->cus);
     if (workspace && pl.ws_bytes > 0) {

@@ -1,0 +1,125 @@
+"""Prefill at f32 precision (f32 pages, head_dim other than 128) against the
+oracle's blockwise attention, at the edges of its tiles: columns (query rows
+times the GQA group) around a wave's 32 and a workgroup's 32 to 128, keys around
+the 32- to 128-key tiles, head_dim below each built size, and launches whose
+waves share a column set's keys four, two and one ways."""
+import numpy as np
+import pytest
+
+import airkv
+from airkv import workloads
+from gpu_helpers import log, rel_err, torch_mod
+from test_gpu_prefill import _prefill_case, _setup
+
+pytestmark = pytest.mark.gpu
+
+# Both sides sum in f32 in orders of their own: at most n * 2^-24 apart for n
+# <= 840 keys (5e-5) relative to the largest output; twice that covers the
+# scores' own rounding.
+TOL_F32 = 1e-4
+
+
+# (dtype, head_dim, kv heads, group, block size, query lengths, contexts)
+CASES = [
+    # few columns, long prefixes: four key shares (two from 97 elements on, one
+    # for f32 / 1-byte pages past 128)
+    (dt, d, 1, 8, 16, [1, 4, 5, 2], [701, 64 + 4, 840, 129]) for dt, d in
+    [(airkv.BF16, 64), (airkv.BF16, 96), (airkv.BF16, 256), (airkv.F32, 64), (airkv.F32, 96), (airkv.F32, 128),
+     (airkv.F32, 256), (airkv.INT8, 64), (airkv.FP8, 96), (airkv.INT8, 256)]
+] + [
+    # whole workgroups and one column more, no prefix and ragged ones
+    (dt, d, 4, 4, 32, [31, 32, 33, 97, 128, 1, 200], [31, 32 + 31, 33 + 65, 97, 128 + 256, 300, 200]) for dt, d in
+    [(airkv.BF16, 32), (airkv.BF16, 64), (airkv.BF16, 96), (airkv.BF16, 160), (airkv.BF16, 256), (airkv.F32, 64),
+     (airkv.F32, 128), (airkv.F32, 224), (airkv.FP8, 64), (airkv.INT8, 96)]
+] + [
+    # columns that are no multiple of the group's rows, one head per kv head,
+    # a group above the vector kernel's eight heads
+    (airkv.BF16, 64, 8, 7, 16, [63, 64, 65, 130, 9, 300], [63, 64 + 1, 65 + 400, 130, 9 + 77, 300]),
+    (airkv.F32, 64, 8, 1, 16, [255, 257, 129, 511, 1, 37], [255, 257 + 9, 129, 511, 1, 400]),
+    (airkv.F32, 128, 2, 12, 16, [90, 170], [90, 170 + 33]),
+]
+
+
+@pytest.mark.parametrize("q_bf16", [True, False])
+@pytest.mark.parametrize("dtype,d,n_kv,group,bs,q_lens,ctx", CASES)
+def test_prefill_f32_tile_edges(dtype, d, n_kv, group, bs, q_lens, ctx, q_bf16):
+    cfg = workloads.Config("f32", n_kv * group, n_kv, d, bs, dtype, len(ctx))
+    got, want = _prefill_case(cfg, ctx, q_lens, seed=31 + d + group, q_bf16=q_bf16)
+    err = rel_err(got, want)
+    log(f"prefill f32 dtype={dtype} d={d} group={group} q_bf16={q_bf16}: rel err {err:.2e}")
+    assert err <= TOL_F32
+
+
+@pytest.mark.parametrize("dtype,d", [(airkv.BF16, 64), (airkv.F32, 64), (airkv.F32, 128)])
+def test_prefill_f32_non_finite_values_stay_behind_the_mask(dtype, d):
+    """Non-finite elements of a value row reach the query rows that see that
+    token, in their own channels; every other output is as with finite ones."""
+    torch = torch_mod()
+    n_kv, group, bs, n = 4, 4, 16, 200
+    cfg = workloads.Config("inf", n_kv * group, n_kv, d, bs, dtype, 2)
+    pool, host, tables, lens = _setup(cfg, [n, n], seed=5)
+    at = 150                                             # token of sequence 0 that turns non-finite
+    slot = np.array([tables[0, at // bs] * bs + at % bs], np.int64)
+    k = np.random.default_rng(1).standard_normal((1, n_kv, d)).astype(np.float32)
+    v = k.copy()
+    v[0, :, [3, d - 1]] = 0.0
+    host.append(k, v, slot)
+    v[0, :, 3], v[0, :, d - 1] = np.inf, np.nan
+    pool.append(torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda(), torch.from_numpy(slot).cuda())
+    cu = np.array([0, n, 2 * n], np.int32)
+    q = np.random.default_rng(2).standard_normal((2 * n, cfg.n_q_heads, d)).astype(np.float32)
+    out = torch.empty(q.shape, device="cuda")
+    pool.paged_prefill(torch.from_numpy(q).cuda(), torch.from_numpy(cu).cuda(), torch.from_numpy(tables).cuda(),
+                       torch.from_numpy(lens).cuda(), out)
+    torch.cuda.synchronize()
+    got, want = out.cpu().numpy(), host.paged_prefill(q, cu, tables, lens)
+    assert np.isposinf(got[at:n, :, 3]).all() and np.isnan(got[at:n, :, d - 1]).all()
+    got[at:n, :, [3, d - 1]] = want[at:n, :, [3, d - 1]]
+    assert np.isfinite(got).all()
+    assert rel_err(got, want) <= TOL_F32
+
+
+def test_prefill_f32_invalid_sequences():
+    """A chunk longer than its sequence and a seq_len beyond the table are each
+    counted once with their rows zero-filled; an out-of-pool table entry is
+    counted once and read as zero keys and values; rows outside every sequence
+    keep their bytes."""
+    torch = torch_mod()
+    cfg = workloads.Config("bad", 32, 8, 64, 16, airkv.BF16, 3)
+    pool, host, tables, lens = _setup(cfg, [400, 300, 350], seed=79)
+    q_lens = [200, 301, 100]
+    lens_bad = lens.copy()
+    lens_bad[2] = tables.shape[1] * 16 + 1
+    cu = np.zeros(4, np.int32)
+    cu[1:] = np.cumsum(q_lens)
+    total = int(cu[-1])
+    q = torch.randn((total + 3, 32, 64), device="cuda")
+    out = torch.full((total + 3, 32, 64), 7.0, device="cuda")
+    args = (torch.from_numpy(cu).cuda(), torch.from_numpy(tables).cuda())
+    pool.error_count(reset=True)
+    pool.paged_prefill(q, *args, torch.from_numpy(lens_bad).cuda(), out)
+    torch.cuda.synchronize()
+    assert pool.error_count(reset=True) == 2
+    got = out.cpu().numpy()
+    assert np.all(got[200:total] == 0.0) and np.all(got[total:] == 7.0)
+    want = host.paged_prefill(q.cpu().numpy()[:200], cu[:2], tables[:1], lens[:1])
+    assert rel_err(got[:200], want) <= TOL_F32
+    # an out-of-pool entry: as a block of zeros
+    t2 = tables.copy()
+    t2[0, 3] = pool.num_blocks + 5
+    hz = _host_with_zero_block(host, cfg)
+    t3 = tables.copy()
+    t3[0, 3] = host.num_blocks
+    out.fill_(7.0)
+    pool.paged_prefill(q, args[0], torch.from_numpy(t2).cuda(), torch.from_numpy(lens_bad).cuda(), out)
+    torch.cuda.synchronize()
+    assert pool.error_count(reset=True) == 3
+    want = hz.paged_prefill(q.cpu().numpy()[:200], cu[:2], t3[:1], lens[:1])
+    assert rel_err(out.cpu().numpy()[:200], want) <= TOL_F32
+
+
+def _host_with_zero_block(host, cfg):
+    import oracle
+    hz = oracle.HostPool(host.num_blocks + 1, cfg.block_size, cfg.n_kv_heads, cfg.head_dim, cfg.dtype)
+    hz.k[:host.num_blocks], hz.v[:host.num_blocks] = host.k, host.v
+    return hz
