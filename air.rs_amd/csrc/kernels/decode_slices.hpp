@@ -1,0 +1,188 @@
+// The balanced-slice work division shared by the decode kernels (described at
+// paged_decode_mfma.hip): the batch's 16-token tiles numbered sequence after
+// sequence, cut into equal contiguous slices, one wave each.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "decode_common.hpp"
+
+namespace airkv {
+
+constexpr int kSliceThreads = 256;         // threads of every workgroup that calls these
+constexpr int kMaxBatch = 4096;            // sequences per launch (the host splits larger batches)
+
+// Reductions across the lanes 16 and 32 apart with the gfx950 lane-swap
+// instructions instead of LDS permutes.  permlane16_swap(v, v) returns
+// {v[l & ~16], v[l | 16]} in lane l, permlane32_swap(v, v) returns
+// {v[l & ~32], v[l | 32]}: the two halves of each pair, in the same order
+// in both lanes, so both lanes compute the same bits.
+__device__ __forceinline__ float max_x16(float x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float max_x32(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float sum_x16(float x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float sum_x32(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// Register-pair transposes: afterwards x_b in lane l holds what x_c held in
+// lane l', where c is lane l's bit 3 (bit 5) and l' is l with that bit set
+// to b.  Bit 3: DPP row_ror:8 (lane l ^ 8 within each row of 16), written
+// only to the lanes whose bit 3 differs from the register index (bank masks
+// 0xC: lanes 8..15 of each row, 0x3: lanes 0..7).  Bit 5: the lane swap
+// across the wave's halves.
+__device__ __forceinline__ void swap_lane_bit3(u32x4 &x0, u32x4 &x1) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int a = (int)x0[j], b = (int)x1[j];
+        x0[j] = (uint32_t)__builtin_amdgcn_update_dpp(a, b, 0x128, 0xF, 0xC, false);
+        x1[j] = (uint32_t)__builtin_amdgcn_update_dpp(b, a, 0x128, 0xF, 0x3, false);
+    }
+}
+__device__ __forceinline__ void swap_lane_bit5(u32x4 &x0, u32x4 &x1) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const auto r = __builtin_amdgcn_permlane32_swap(x0[j], x1[j], false, false);
+        x0[j] = r[0];
+        x1[j] = r[1];
+    }
+}
+
+__device__ __forceinline__ int64_t clamp_len(int64_t len, int64_t max_len) {
+    return len < 0 ? 0 : (len > max_len ? max_len : len);
+}
+
+// Tiles per slice: an equal share of `total`, at least min_chunk, and large
+// enough that no sequence is cut into more than max_splits pieces.  A
+// sequence of T tiles starting anywhere meets at most ceil((T - 1) / chunk) +
+// 1 slices, so chunk >= ceil((T - 1) / (max_splits - 1)) for the longest
+// sequence (tmax tiles) bounds every one; max_splits 1 leaves one slice per
+// kv head.
+__device__ __forceinline__ int slice_chunk(int total, int slices, int tmax, int max_splits,
+                                           int min_chunk) {
+    int c = (total + slices - 1) / slices;
+    c = c < min_chunk ? min_chunk : c;
+    if (max_splits <= 1) return c > total ? c : total;
+    const int cs = (tmax - 1 + max_splits - 2) / (max_splits - 1);
+    return c > cs ? c : cs;
+}
+
+// Inclusive sum / running maximum over a wave's lanes (DPP: row shifts, then
+// the rows' last lanes broadcast; the identity of both is 0).
+template <class F> __device__ __forceinline__ int wave_scan(int x, F f) {
+    x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false));   // row_shr:1
+    x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false));   // row_shr:2
+    x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false));   // row_shr:4
+    x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false));   // row_shr:8
+    x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false));   // row_bcast:15 into rows 1, 3
+    x = f(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false));   // row_bcast:31 into rows 2, 3
+    return x;
+}
+
+// pre[b] = tiles (ceil(len / 16), len clamped to [0, max_blocks * bs]) of the
+// sequences before b, for b = 0..batch, in LDS, and pre[B + 1] = the most
+// tiles of one sequence.  All threads take part.
+// long_seq (optional, ceil(B / 32) words): bit b set when sequence b is longer
+// than its table, else clear.
+//
+// Up to 64 sequences are one lane each: every wave scans them in registers and
+// writes the same values, which it alone reads, so the launch's first loads
+// are not held up by the workgroup's barriers.
+__device__ __forceinline__ void tile_prefix(const DecodeArgs &a, int bs, int32_t *pre, int32_t *wsum,
+                                            uint32_t *long_seq = nullptr) {
+    if (a.batch <= 64) {
+        const int lane = threadIdx.x & 63;
+        const int64_t max_len = (int64_t)a.max_blocks * bs;
+        const int32_t len = lane < a.batch ? a.lens[lane] : 0;
+        const int32_t t = (int32_t)((clamp_len(len, max_len) + 15) / 16);
+        const int incl = wave_scan(t, [](int x, int y) { return x + y; });
+        const int most = wave_scan(t, [](int x, int y) { return x > y ? x : y; });
+        if (lane < a.batch) pre[lane + 1] = incl;
+        if (lane == 63) {
+            pre[0] = 0;
+            pre[a.batch + 1] = most;
+        }
+        if (long_seq) {
+            const uint64_t m = __ballot(len > max_len);
+            if (lane < (a.batch + 31) / 32) long_seq[lane] = (uint32_t)(lane ? m >> 32 : m);
+        }
+        return;
+    }
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int B = a.batch;
+    const int64_t max_len = (int64_t)a.max_blocks * bs;
+    if (long_seq) {
+        for (int i = tid; i < (B + 31) / 32; i += kSliceThreads) long_seq[i] = 0;
+        __syncthreads();
+    }
+    int tmax = 0;
+    for (int b = tid; b < B; b += kSliceThreads) {
+        const int32_t len = a.lens[b];
+        const int32_t t = (int32_t)((clamp_len(len, max_len) + 15) / 16);
+        pre[b + 1] = t;
+        tmax = t > tmax ? t : tmax;
+        if (long_seq && len > max_len) atomicOr(&long_seq[b >> 5], 1u << (b & 31));
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const int y = __shfl_xor(tmax, o);
+        tmax = y > tmax ? y : tmax;
+    }
+    if (lane == 0) wsum[wave] = tmax;
+    if (tid == 0) pre[0] = 0;
+    __syncthreads();
+    if (tid == 0) {
+        int m = wsum[0];
+        for (int w = 1; w < kSliceThreads / 64; ++w) m = wsum[w] > m ? wsum[w] : m;
+        pre[B + 1] = m;
+    }
+    __syncthreads();
+    // each thread scans a run of `per` entries; runs are chained by a
+    // wave-level then a workgroup-level exclusive scan of the run sums
+    const int per = (B + kSliceThreads - 1) / kSliceThreads;
+    const int lo = 1 + tid * per;
+    const int hi = lo + per < B + 1 ? lo + per : B + 1;
+    int sum = 0;
+    for (int i = lo; i < hi; ++i) sum += pre[i];
+    int incl = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(incl, o);
+        if (lane >= o) incl += y;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int run = incl - sum;
+    for (int w = 0; w < wave; ++w) run += wsum[w];
+    for (int i = lo; i < hi; ++i) {
+        run += pre[i];
+        pre[i] = run;
+    }
+    __syncthreads();
+}
+
+// The sequence holding tile t (0 <= t < pre[B]): the b with pre[b] <= t < pre[b + 1].
+// The loop count depends on B only, so the lanes of a wave stay converged.
+__device__ __forceinline__ int seq_of_tile(const int32_t *pre, int B, int t) {
+    int lo = 0, hi = B;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (pre[mid] <= t) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+}  // namespace airkv

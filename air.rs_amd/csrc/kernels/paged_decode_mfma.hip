@@ -48,6 +48,7 @@
 #include "../pool.hpp"
 #include "codecs.hpp"
 #include "decode_common.hpp"
+#include "decode_slices.hpp"
 #include "page_io.hpp"
 
 namespace airkv {
@@ -59,9 +60,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kThreads = 256;
+constexpr int kThreads = kSliceThreads;
 constexpr int kWaves = kThreads / 64;
-constexpr int kMaxBatch = 4096;            // sequences per launch (the host splits larger batches)
 constexpr int kMinChunk = 4;               // tiles per slice at least
 
 // Build-time tuning knobs (defaults are the shipped configuration).
@@ -148,51 +148,6 @@ __device__ __forceinline__ uint32_t bf16_pair(float x, float y) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x, y}), bf16x2));
 }
 
-// Reductions across the lanes 16 and 32 apart with the gfx950 lane-swap
-// instructions instead of LDS permutes.  permlane16_swap(v, v) returns
-// {v[l & ~16], v[l | 16]} in lane l, permlane32_swap(v, v) returns
-// {v[l & ~32], v[l | 32]}: the two halves of each pair, in the same order
-// in both lanes, so both lanes compute the same bits.
-__device__ __forceinline__ float max_x16(float x) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float max_x32(float x) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float sum_x16(float x) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float sum_x32(float x) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// Register-pair transposes: afterwards x_b in lane l holds what x_c held in
-// lane l', where c is lane l's bit 3 (bit 5) and l' is l with that bit set
-// to b.  Bit 3: DPP row_ror:8 (lane l ^ 8 within each row of 16), written
-// only to the lanes whose bit 3 differs from the register index (bank masks
-// 0xC: lanes 8..15 of each row, 0x3: lanes 0..7).  Bit 5: the lane swap
-// across the wave's halves.
-__device__ __forceinline__ void swap_lane_bit3(u32x4 &x0, u32x4 &x1) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int a = (int)x0[j], b = (int)x1[j];
-        x0[j] = (uint32_t)__builtin_amdgcn_update_dpp(a, b, 0x128, 0xF, 0xC, false);
-        x1[j] = (uint32_t)__builtin_amdgcn_update_dpp(b, a, 0x128, 0xF, 0x3, false);
-    }
-}
-__device__ __forceinline__ void swap_lane_bit5(u32x4 &x0, u32x4 &x1) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const auto r = __builtin_amdgcn_permlane32_swap(x0[j], x1[j], false, false);
-        x0[j] = r[0];
-        x1[j] = r[1];
-    }
-}
-
 __device__ __forceinline__ void store_out(const DecodeArgs &a, int64_t idx, float v) {
     if (a.out_dtype == AIR_KV_F32) ((float *)a.out)[idx] = v;
     else ((uint16_t *)a.out)[idx] = bf16_rne(v);
@@ -207,92 +162,6 @@ __device__ __forceinline__ void store_out4(const DecodeArgs &a, int64_t idx, f32
                          (uint32_t)bf16_rne(v[2]) | ((uint32_t)bf16_rne(v[3]) << 16)};
         *reinterpret_cast<u32x2 *>((uint16_t *)a.out + idx) = w;
     }
-}
-
-__device__ __forceinline__ int64_t clamp_len(int64_t len, int64_t max_len) {
-    return len < 0 ? 0 : (len > max_len ? max_len : len);
-}
-
-// Tiles per slice: an equal share of `total`, at least kMinChunk, and large
-// enough that no sequence is cut into more than max_splits pieces.  A
-// sequence of T tiles starting anywhere meets at most ceil((T - 1) / chunk) +
-// 1 slices, so chunk >= ceil((T - 1) / (max_splits - 1)) for the longest
-// sequence (tmax tiles) bounds every one; max_splits 1 leaves one slice per
-// kv head.
-__device__ __forceinline__ int slice_chunk(int total, int slices, int tmax, int max_splits) {
-    int c = (total + slices - 1) / slices;
-    c = c < kMinChunk ? kMinChunk : c;
-    if (max_splits <= 1) return c > total ? c : total;
-    const int cs = (tmax - 1 + max_splits - 2) / (max_splits - 1);
-    return c > cs ? c : cs;
-}
-
-// pre[b] = tiles (ceil(len / 16), len clamped to [0, max_blocks * BS]) of the
-// sequences before b, for b = 0..batch, in LDS, and pre[B + 1] = the most
-// tiles of one sequence.  All threads take part.
-template <int BS>
-// long_seq (optional, B bits, zero on entry): bit b set when sequence b is
-// longer than its table.
-__device__ void tile_prefix(const DecodeArgs &a, int32_t *pre, int32_t *wsum, uint32_t *long_seq = nullptr) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int B = a.batch;
-    const int64_t max_len = (int64_t)a.max_blocks * BS;
-    int tmax = 0;
-    for (int b = tid; b < B; b += kThreads) {
-        const int32_t len = a.lens[b];
-        const int32_t t = (int32_t)((clamp_len(len, max_len) + 15) / 16);
-        pre[b + 1] = t;
-        tmax = t > tmax ? t : tmax;
-        if (long_seq && len > max_len) atomicOr(&long_seq[b >> 5], 1u << (b & 31));
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const int y = __shfl_xor(tmax, o);
-        tmax = y > tmax ? y : tmax;
-    }
-    if (lane == 0) wsum[wave] = tmax;
-    if (tid == 0) pre[0] = 0;
-    __syncthreads();
-    if (tid == 0) {
-        int m = wsum[0];
-        for (int w = 1; w < kWaves; ++w) m = wsum[w] > m ? wsum[w] : m;
-        pre[B + 1] = m;
-    }
-    __syncthreads();
-    // each thread scans a run of `per` entries; runs are chained by a
-    // wave-level then a workgroup-level exclusive scan of the run sums
-    const int per = (B + kThreads - 1) / kThreads;
-    const int lo = 1 + tid * per;
-    const int hi = lo + per < B + 1 ? lo + per : B + 1;
-    int sum = 0;
-    for (int i = lo; i < hi; ++i) sum += pre[i];
-    int incl = sum;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(incl, o);
-        if (lane >= o) incl += y;
-    }
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    int run = incl - sum;
-    for (int w = 0; w < wave; ++w) run += wsum[w];
-    for (int i = lo; i < hi; ++i) {
-        run += pre[i];
-        pre[i] = run;
-    }
-    __syncthreads();
-}
-
-// The sequence holding tile t (0 <= t < pre[B]): the b with pre[b] <= t < pre[b + 1].
-// The loop count depends on B only, so the lanes of a wave stay converged.
-__device__ __forceinline__ int seq_of_tile(const int32_t *pre, int B, int t) {
-    int lo = 0, hi = B;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (pre[mid] <= t) lo = mid;
-        else hi = mid;
-    }
-    return lo;
 }
 
 // Raw registers of one 16-token tile as loaded, before any conversion.
@@ -423,15 +292,13 @@ void decode_mfma_kernel(DecodeArgs a) {
     // fused append: sequences longer than their table (they append nothing)
     __shared__ uint32_t s_long[APPEND ? kMaxBatch / 32 : 1];
     if constexpr (APPEND) {
-        for (int i = threadIdx.x; i < (a.batch + 31) / 32; i += kThreads) s_long[i] = 0;
-        __syncthreads();
-        tile_prefix<BS>(a, s_pre, s_wsum, s_long);
+        tile_prefix(a, BS, s_pre, s_wsum, s_long);
     } else {
-        tile_prefix<BS>(a, s_pre, s_wsum);
+        tile_prefix(a, BS, s_pre, s_wsum);
     }
     const int B = a.batch;
     const int total = s_pre[B];
-    const int chunk = slice_chunk(total, a.slices, s_pre[B + 1], a.max_splits);
+    const int chunk = slice_chunk(total, a.slices, s_pre[B + 1], a.max_splits, kMinChunk);
     if (blockIdx.x == 0) {                     // for the merge kernel: prefix, then the chunk
         for (int i = threadIdx.x; i <= B; i += kThreads) a.prefix[i] = s_pre[i];
         if (threadIdx.x == 0) a.prefix[B + 1] = chunk;
@@ -1160,7 +1027,6 @@ int plan_decode_mfma(const air_kv_pool &p, int32_t n_q_heads, int32_t batch, int
     const int64_t slices = slices_for(waves_per_simd(p.desc.dtype));
     plan->mfma = true;
     plan->dtype = p.desc.dtype;
-    plan->part_tokens = plan->num_parts = 0;
     plan->slices = (int32_t)slices;
     // the f32-query build's slices (what is resident at once; the workspace,
     // sized for plan->slices, holds them whenever that build runs fewer waves)

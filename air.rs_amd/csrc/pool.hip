@@ -260,9 +260,7 @@ int air_paged_prefill(air_kv_pool *p, void *stream, const void *q, int32_t q_dty
         if (batch > 65535) return fail(AIR_KV_E_INVALID_ARG, "batch %d above 65535 for this pool", batch);
         hipError_t e = airkv::prefill_f32_better(a, d.dtype, max_q_len)
                            ? airkv::launch_prefill_f32(a, d.dtype, max_q_len, p->cus, (hipStream_t)stream)
-                           : airkv::launch_prefill_rows(*p, (hipStream_t)stream, q, q_dtype, n_q_heads, cu_q, total_q,
-                                                        max_q_len, block_tables, seq_lens, batch, max_blocks, scale,
-                                                        out, out_dtype);
+                           : airkv::launch_prefill_rows(a, d.dtype, max_q_len, (hipStream_t)stream);
         return e == hipSuccess ? AIR_KV_OK : hip_fail(e, "air_paged_prefill launch");
     }
     const airkv::PrefillPlan pl =

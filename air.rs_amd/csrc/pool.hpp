@@ -35,11 +35,7 @@ inline bool dtype_quantized(int dt) { return dt == AIR_KV_INT8 || dt == AIR_KV_F
 struct DecodePlan {
     int32_t group;        // q heads per kv head
     int32_t dtype;        // page dtype of the pool
-    bool mfma;            // matrix-core kernel with balanced slices (else fixed partitions)
-    // fixed partitions (vector kernel)
-    int32_t part_tokens;  // tokens per split-K partition (multiple of block_size)
-    int32_t num_parts;    // partitions per sequence
-    // balanced slices (matrix-core kernel)
+    bool mfma;            // paged_decode_mfma.hip (else paged_decode_f32.hip)
     int32_t slices;       // slices per kv head (one wave each)
     int32_t slices_qf32;  // the same for f32 queries (their kernel may hold fewer waves per SIMD)
     int32_t slices_append;  // the same for the fused append + decode
@@ -62,12 +58,6 @@ hipError_t launch_decode(const air_kv_pool &pool, hipStream_t s, const DecodePla
                          const int32_t *lens, int32_t batch, int32_t max_blocks, float scale,
                          void *workspace, void *out, int32_t out_dtype,
                          const float *k_new = nullptr, const float *v_new = nullptr);
-// Paged prefill on the vector decode kernel, for pools the matrix-core
-// prefill does not take (arguments as air_paged_prefill's, validated).
-hipError_t launch_prefill_rows(const air_kv_pool &pool, hipStream_t s, const void *q, int32_t q_dtype,
-                               int32_t n_q_heads, const int32_t *cu_q, int32_t total_q, int32_t max_q_len,
-                               const int32_t *tables, const int32_t *lens, int32_t batch, int32_t max_blocks,
-                               float scale, void *out, int32_t out_dtype);
 hipError_t launch_copy_blocks(const air_kv_pool &pool, hipStream_t s, const int32_t *src,
                               const int32_t *dst, int32_t n);
 hipError_t launch_stage_blocks(const air_kv_pool &pool, hipStream_t s, const int32_t *ids, int32_t n,

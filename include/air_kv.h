@@ -244,26 +244,25 @@ int air_paged_decode_workspace_size(const air_kv_pool *pool, int32_t n_q_heads, 
 /* Split-K paged decode attention for one new token per sequence:
  *   out[b][h] = softmax(q[b][h] . K_b[h / group]^T * scale) . V_b[h / group]
  * over all seq_lens[b] cached tokens, group = n_q_heads / n_kv_heads (the GQA
- * map of src/chunked_attn.rs:240-243).  Replaces ops::attention for seq_q = 1
- * (src/ops.rs:333-357, :514-568) and generalises flash_decode
- * (src/flash_decode.rs:153-173: split-K partials merged by log-sum-exp,
- * :114-142) to paged storage.  q: [batch][n_q_heads][head_dim] as q_dtype
+ * map of src/chunked_attn.rs:240-243; any ratio, :65-72).  Replaces
+ * ops::attention for seq_q = 1 (src/ops.rs:333-357, :514-568) and generalises
+ * flash_decode (src/flash_decode.rs:153-173: split-K partials merged by
+ * log-sum-exp, :114-142) to paged storage.  q: [batch][n_q_heads][head_dim] as q_dtype
  * (AIR_KV_F32 or AIR_KV_BF16); out likewise as out_dtype.  On the
  * matrix-core kernel F32 queries enter the products as two bf16 halves on
  * BF16 pools and rounded to bf16 on INT8 / FP8 pools (an error an order below
  * their quantization's).  The reference's
  * scale is 1/sqrt(head_dim).  max_splits (1..256) bounds the split-K work
- * division: no sequence is cut into more than max_splits partitions.  Pools
- * with head_dim 128, block_size 16 or 32 and group 1..16 -- bf16, and int8 /
- * fp8 with scale_group >= 32 -- take the matrix-core kernel, which cuts the
- * batch's cached tokens into equal slices per kv head (one wave each, at most
- * batch * max_splits), where a slice may end inside a sequence and hold
+ * division: no sequence is cut into more than max_splits partitions.  The
+ * batch's cached tokens are cut into equal slices per kv head (one wave each,
+ * at most batch * max_splits), where a slice may end inside a sequence and hold
  * several, widened when the longest sequence would otherwise meet more than
- * max_splits of them (max_splits 1: one slice per kv head); other pools
- * (F32 pages, head_dim 64 or 256, groups above 16) cut each sequence into at
- * most max_splits fixed partitions, each workgroup serving up to 8 query
- * heads of a kv head (any group: the reference's head map takes any
- * n_q_heads / n_kv_heads, src/chunked_attn.rs:65-72).  Out-of-pool table
+ * max_splits of them (max_splits 1: one slice per kv head).  Pools with
+ * head_dim 128, block_size 16 or 32 and group 1..16 -- bf16, and int8 / fp8
+ * with scale_group >= 32 -- take a kernel with 16-bit operands; other pools
+ * (F32 pages, other head dims, groups above 16, small scale groups) one that
+ * keeps queries, keys, probabilities and values at f32 precision, 16 query
+ * heads of a kv head to a wave.  Out-of-pool table
  * entries are skipped and counted (air_kv_pool_error_count); seq_lens outside
  * [0, max_blocks * block_size] are clamped and counted.  A sequence of length
  * 0 produces zeros.  The workspace is device
@@ -284,14 +283,10 @@ int air_paged_decode(air_kv_pool *pool, void *stream, const void *q, int32_t q_d
  * the wave that attends over it, so no launch orders the two.  Sequences of
  * length 0 append nothing; a sequence longer than its table, or whose last
  * block is outside the pool, appends nothing and is counted as by
- * air_paged_decode.  On the matrix-core decode (head_dim 128, block_size 16
- * or 32, group 1..16; BF16, or INT8 / FP8 with scale_group >= 32, whose new
- * rows are quantized exactly as air_kv_append quantizes them: the same codes
- * and group scales) this is one launch; every other pool takes the same
- * call as three launches on the stream (each sequence's slot from its
- * table, air_kv_append's kernel, then the decode), with the same pages and
- * outputs.  k_new and v_new are 16-byte aligned device pointers.  The
- * workspace is air_paged_decode's. */
+ * air_paged_decode.  New rows of INT8 / FP8 pools are quantized exactly as
+ * air_kv_append quantizes them: the same codes and group scales.  k_new and
+ * v_new are 16-byte aligned device pointers.  The workspace is
+ * air_paged_decode's. */
 int air_paged_decode_append(air_kv_pool *pool, void *stream, const void *q, int32_t q_dtype,
                             int32_t n_q_heads, const float *k_new, const float *v_new,
                             const int32_t *block_tables, const int32_t *seq_lens, int32_t batch,
@@ -339,7 +334,7 @@ int air_paged_decode_noalloc(air_kv_pool *pool, void *stream, const void *q, int
  * 128 take the matrix-core kernel (quantized pages are dequantized q * scale
  * in registers); every other pool (F32 pages, other head dims) keeps queries,
  * keys, probabilities and values at f32 precision, on the matrix cores or, for
- * launches too small for them, on air_paged_decode's split kernel, without a
+ * launches too small for them, row by row on the vector ALUs, without a
  * workspace and with the same error handling.  BF16 pools of 128 run the probability x value
  * products with f16 operands (11 significant bits each), INT8 / FP8 pools the
  * key x query products as well (keys, values and F32 queries rounded to f16

@@ -1,0 +1,101 @@
+"""Decode at f32 precision (f32 pages, head_dim other than 128, small scale
+groups, GQA groups above 16) against the oracle's gather + flash_decode, at the
+edges of its tiles: sequences around its 16-token tiles and the 64-tile windows
+of a slice, head_dim below each built size, groups around its 16 heads, batches
+on both sides of the 64 sequences one wave scans, and the step's appended row."""
+import numpy as np
+import pytest
+
+import airkv
+from airkv import workloads
+from gpu_helpers import log, rel_err, torch_mod
+from test_gpu_decode import _decode_case
+from test_gpu_decode_append import _run_pair, _setup
+
+pytestmark = pytest.mark.gpu
+
+# Both sides sum in f32 in orders of their own: at most n * 2^-24 apart for n
+# <= 1100 keys (6.6e-5) relative to the largest output; half as much again
+# covers the scores' own rounding.
+TOL_F32 = 1e-4
+
+LENS = [0, 14, 15, 16, 30, 31, 32, 62, 63, 64, 1, 255, 1022, 1024, 333]      # + 1 token each
+
+
+# (dtype, head_dim, kv heads, group, block size, scale group, sequences)
+CASES = [(dt, d, 2, 4, 16, 32, 15) for dt in (airkv.F32, airkv.BF16, airkv.INT8, airkv.FP8)
+         for d in (32, 64, 96, 160, 256)] + [
+    (airkv.F32, 128, 8, 1, 32, 32, 15), (airkv.F32, 128, 1, 17, 16, 32, 15), (airkv.BF16, 128, 1, 40, 32, 32, 15),
+    (airkv.INT8, 128, 2, 7, 16, 16, 15), (airkv.FP8, 64, 2, 16, 32, 8, 15), (airkv.BF16, 224, 2, 16, 32, 32, 15),
+    (airkv.BF16, 64, 8, 4, 16, 32, 65), (airkv.F32, 64, 4, 2, 16, 32, 130), (airkv.INT8, 96, 1, 3, 32, 32, 64),
+]
+
+
+@pytest.mark.parametrize("q_bf16", [True, False])
+@pytest.mark.parametrize("dtype,d,n_kv,group,bs,scale_group,batch", CASES)
+def test_decode_f32_tile_edges(dtype, d, n_kv, group, bs, scale_group, batch, q_bf16):
+    lens = (LENS * (batch // len(LENS) + 1))[:batch]
+    cfg = workloads.Config("f32", n_kv * group, n_kv, d, bs, dtype, batch, scale_group=scale_group)
+    got, want, (pool, host, tables, seq_lens, q, _) = _decode_case(cfg, lens, seed=13 + d + group, q_bf16=q_bf16)
+    err = rel_err(got, want)
+    # the same sequences in few, long slices, and in one
+    torch = torch_mod()
+    qt = torch.from_numpy(q).cuda()
+    qt = qt.to(torch.bfloat16) if q_bf16 else qt
+    for most in (1, 2, 7):
+        out = torch.full(q.shape, float("nan"), device="cuda")
+        pool.paged_decode(qt, torch.from_numpy(tables).cuda(), torch.from_numpy(seq_lens).cuda(), out, max_splits=most)
+        err = max(err, rel_err(out.cpu().numpy(), want))
+    log(f"decode f32 dtype={dtype} d={d} group={group} q_bf16={q_bf16}: rel err {err:.2e}")
+    assert err <= TOL_F32
+    assert pool.error_count() == 0
+
+
+@pytest.mark.parametrize("dtype,d,n_q,scale_group", [(airkv.F32, 256, 20, 32), (airkv.BF16, 96, 7, 32),
+                                                     (airkv.INT8, 160, 34, 32), (airkv.FP8, 32, 8, 8)])
+def test_decode_f32_append_rows(dtype, d, n_q, scale_group):
+    """The appended row at every place of a tile, 70 sequences: pages, scales
+    and outputs equal append, then decode."""
+    ctx = [i % 35 for i in range(70)]
+    cfg = workloads.Config("f32", n_q, 1, d, 16, dtype, len(ctx), scale_group=scale_group)
+    w, pa, pb, host, tables, lens, k_new, v_new = _setup(cfg, ctx, seed=7 + d)
+    q = np.random.default_rng(8).standard_normal((len(ctx), n_q, d)).astype(np.float32)
+    q, got = _run_pair(cfg, pa, pb, host, tables, lens, k_new, v_new, q, q_f32=True)
+    assert rel_err(got, host.paged_decode(q, tables, lens, chunk=64)) <= TOL_F32
+
+
+@pytest.mark.parametrize("d", [64, 96])
+def test_decode_f32_every_fp8_code(d):
+    """Pages written as raw blocks may hold any code: subnormal ones, which the
+    format reads as zero, and 0xFF, which it reads as -480 (0x7F, NaN, is left
+    out), here in single tiles of a sequence; and an entry outside the pool is
+    skipped and counted."""
+    torch = torch_mod()
+    n, bs, kv, group = 1000, 16, 2, 4
+    cfg = workloads.Config("codes", kv * group, kv, d, bs, airkv.FP8, 1)
+    w, pool, _, host, tables, lens, _, _ = _setup(cfg, [n - 1], seed=3)
+    rng = np.random.default_rng(4)
+    for x in (host.k, host.v):
+        codes = np.arange(256, dtype=np.uint8)
+        x[:] = rng.choice(codes[(codes != 0x7F) & (codes != 0xFF)], x.shape)
+        for b in (3, 17):
+            x[tables[0, b]] = rng.choice(codes[codes != 0x7F], x[tables[0, b]].shape)
+            x[tables[0, b], 0, 5, 1] = 0xFF
+    for s in (host.k_scales, host.v_scales):
+        s[:] = rng.uniform(1e-4, 1e-3, s.shape).astype(np.float32)
+    raw = [np.ascontiguousarray(x).reshape(pool.num_blocks, -1).view(np.uint8)
+           for x in (host.k, host.v, host.k_scales, host.v_scales)]
+    pool.write_blocks(np.arange(pool.num_blocks, dtype=np.int32), np.concatenate(raw, 1))
+    lens = np.array([n], np.int32)
+    q = rng.standard_normal((1, kv * group, d)).astype(np.float32)
+    out = torch.empty(q.shape, device="cuda")
+    pool.paged_decode(torch.from_numpy(q).cuda(), torch.from_numpy(tables).cuda(), torch.from_numpy(lens).cuda(), out)
+    want = host.paged_decode(q, tables, lens, chunk=64)
+    assert np.isfinite(want).all() and rel_err(out.cpu().numpy(), want) <= TOL_F32
+    # the last block's entry outside the pool: as if the sequence ended before it
+    assert pool.error_count(reset=True) == 0
+    tables[0, n // bs] = pool.num_blocks + 3
+    pool.paged_decode(torch.from_numpy(q).cuda(), torch.from_numpy(tables).cuda(), torch.from_numpy(lens).cuda(), out)
+    want = host.paged_decode(q, tables, np.array([n // bs * bs], np.int32), chunk=64)
+    assert rel_err(out.cpu().numpy(), want) <= TOL_F32
+    assert pool.error_count(reset=True) > 0
