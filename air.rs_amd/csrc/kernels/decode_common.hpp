@@ -17,6 +17,7 @@ struct DecodeArgs {
     const int32_t *tables, *lens;
     int32_t batch, max_blocks;
     int32_t slices, slots;         // balanced slices per kv head, partial rows per (kv head, query head)
+    int32_t simd_slices;           // slices per kv head that give every SIMD one wave
     int32_t max_splits;            // pieces per sequence at most
     float scale_log2;              // softmax scale * log2(e): exp(x*s) == exp2(x*scale_log2)
     int32_t n_kv_heads, block_size, scale_group, group, head_dim;

@@ -64,16 +64,18 @@ __device__ __forceinline__ int64_t clamp_len(int64_t len, int64_t max_len) {
     return len < 0 ? 0 : (len > max_len ? max_len : len);
 }
 
-// Tiles per slice: an equal share of `total`, at least min_chunk, and large
-// enough that no sequence is cut into more than max_splits pieces.  A
+// Tiles per slice: an equal share of `total` over the resident waves, but at
+// least full_chunk once every SIMD has a wave (simd_slices per kv head), and
+// large enough that no sequence is cut into more than max_splits pieces.  A
 // sequence of T tiles starting anywhere meets at most ceil((T - 1) / chunk) +
 // 1 slices, so chunk >= ceil((T - 1) / (max_splits - 1)) for the longest
 // sequence (tmax tiles) bounds every one; max_splits 1 leaves one slice per
 // kv head.
-__device__ __forceinline__ int slice_chunk(int total, int slices, int tmax, int max_splits,
-                                           int min_chunk) {
+__device__ __forceinline__ int slice_chunk(int total, int slices, int simd_slices, int full_chunk,
+                                           int tmax, int max_splits) {
+    const int lone = (total + simd_slices - 1) / simd_slices;
     int c = (total + slices - 1) / slices;
-    c = c < min_chunk ? min_chunk : c;
+    c = max(c, max(1, min(lone, full_chunk)));
     if (max_splits <= 1) return c > total ? c : total;
     const int cs = (tmax - 1 + max_splits - 2) / (max_splits - 1);
     return c > cs ? c : cs;

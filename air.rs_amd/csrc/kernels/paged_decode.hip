@@ -41,6 +41,8 @@ hipError_t launch_decode(const air_kv_pool &p, hipStream_t s, const DecodePlan &
     a.q = q; a.q_dtype = q_dtype; a.n_q_heads = n_q_heads;
     a.tables = tables; a.lens = lens;
     a.batch = batch; a.max_blocks = max_blocks;
+    const int waves = p.desc.n_kv_heads * ((plan.group + 15) / 16);   // per slice
+    a.simd_slices = (4 * p.cus + waves - 1) / waves;
     a.slices = plan.slices; a.slots = plan.slots; a.max_splits = plan.max_splits;
     a.scale_log2 = scale * 1.4426950408889634f;
     a.n_kv_heads = p.desc.n_kv_heads; a.block_size = p.desc.block_size;

@@ -61,10 +61,11 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = kSliceThreads;
 constexpr int kWaves = kThreads / 64;
-// Tiles per slice at least: a small launch has waves to spare, and one tile
-// more in a wave costs more than one more piece to merge (four sequences of 300
-// tokens, f32 pages of 64, 8 heads: 9.6 us at 1, 11.5 at 2, 14.5 at 4).
-constexpr int kMinChunk = 1;
+// Tiles per slice at least once every SIMD has a wave: these waves' products
+// keep a SIMD less busy than the loads they wait for (64 sequences of 16 to 300
+// tokens, bf16 pages of 64: 13.8 us at one tile, 15.0 at four; 16 of 100 to 800,
+// f32 pages, 14.0 and 15.2).
+constexpr int kFullChunk = 1;
 constexpr int kHeads = 16;                 // query heads of a kv head per wave
 constexpr int kBufferWord3 = 0x00020000;   // raw buffer access
 constexpr int kOutside = 1 << 30;          // a lane offset no page tile reaches: reads as zero
@@ -207,7 +208,7 @@ void decode_f32_kernel(DecodeArgs a) {
     tile_prefix(a, a.block_size, s_pre, s_wsum, s_long);
     const int B = a.batch;
     const int total = s_pre[B];
-    const int chunk = slice_chunk(total, a.slices, s_pre[B + 1], a.max_splits, kMinChunk);
+    const int chunk = slice_chunk(total, a.slices, a.simd_slices, kFullChunk, s_pre[B + 1], a.max_splits);
     if (blockIdx.x == 0) {                     // for the merge kernel: prefix, then the chunk
         for (int i = threadIdx.x; i <= B; i += kThreads) a.prefix[i] = s_pre[i];
         if (threadIdx.x == 0) a.prefix[B + 1] = chunk;

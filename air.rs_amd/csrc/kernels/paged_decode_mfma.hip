@@ -62,7 +62,13 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = kSliceThreads;
 constexpr int kWaves = kThreads / 64;
-constexpr int kMinChunk = 4;               // tiles per slice at least
+// Tiles per slice at least once every SIMD has a wave.  Until then a slice may
+// hold fewer: a tile more in a wave costs more than a piece more to merge (1
+// sequence of 100 tokens, 32 heads over 8, bf16: 8.0 us, 9.8 at four tiles
+// always; 64 of 16 to 64 tokens 10.4, 14.0; 8 of 64 to 512, fp8, 9.5, 12.2).
+// Past it, short slices only add waves that share a SIMD (16 sequences of 100 to
+// 800: 13.2 us, 14.8 at one or two tiles always; 64 of 30 to 300, fp8, 18.3, 20.4).
+constexpr int kFullChunk = 4;
 
 // Build-time tuning knobs (defaults are the shipped configuration).
 #ifndef AIRKV_DECODE_WAVES_PER_EU
@@ -298,7 +304,7 @@ void decode_mfma_kernel(DecodeArgs a) {
     }
     const int B = a.batch;
     const int total = s_pre[B];
-    const int chunk = slice_chunk(total, a.slices, s_pre[B + 1], a.max_splits, kMinChunk);
+    const int chunk = slice_chunk(total, a.slices, a.simd_slices, kFullChunk, s_pre[B + 1], a.max_splits);
     if (blockIdx.x == 0) {                     // for the merge kernel: prefix, then the chunk
         for (int i = threadIdx.x; i <= B; i += kThreads) a.prefix[i] = s_pre[i];
         if (threadIdx.x == 0) a.prefix[B + 1] = chunk;
