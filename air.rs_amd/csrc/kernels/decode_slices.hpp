@@ -99,26 +99,36 @@ template <class F> __device__ __forceinline__ int wave_scan(int x, F f) {
 // long_seq (optional, ceil(B / 32) words): bit b set when sequence b is longer
 // than its table, else clear.
 //
-// Up to 64 sequences are one lane each: every wave scans them in registers and
-// writes the same values, which it alone reads, so the launch's first loads
+// Up to kScanBatch sequences: every wave scans them in registers, 64 at a time,
+// and writes the same values, which it alone reads, so the launch's first loads
 // are not held up by the workgroup's barriers.
 __device__ __forceinline__ void tile_prefix(const DecodeArgs &a, int bs, int32_t *pre, int32_t *wsum,
                                             uint32_t *long_seq = nullptr) {
-    if (a.batch <= 64) {
-        const int lane = threadIdx.x & 63;
+    constexpr int kScanBatch = 256, kSteps = kScanBatch / 64;
+    if (a.batch <= kScanBatch) {
+        const int lane = threadIdx.x & 63, B = a.batch;
         const int64_t max_len = (int64_t)a.max_blocks * bs;
-        const int32_t len = lane < a.batch ? a.lens[lane] : 0;
-        const int32_t t = (int32_t)((clamp_len(len, max_len) + 15) / 16);
-        const int incl = wave_scan(t, [](int x, int y) { return x + y; });
-        const int most = wave_scan(t, [](int x, int y) { return x > y ? x : y; });
-        if (lane < a.batch) pre[lane + 1] = incl;
+        int32_t len[kSteps];
+#pragma unroll
+        for (int k = 0; k < kSteps; ++k) len[k] = 64 * k + lane < B ? a.lens[64 * k + lane] : 0;
+        int before = 0, most = 0;
+#pragma unroll
+        for (int k = 0; k < kSteps; ++k) {
+            if (64 * k >= B) break;
+            const int32_t t = (int32_t)((clamp_len(len[k], max_len) + 15) / 16);
+            const int incl = before + wave_scan(t, [](int x, int y) { return x + y; });
+            if (64 * k + lane < B) pre[64 * k + lane + 1] = incl;
+            before = __builtin_amdgcn_readlane(incl, 63);
+            most = max(most, t);
+            if (long_seq) {
+                const uint64_t m = __ballot(len[k] > max_len);
+                if (lane < 2 && 64 * k + 32 * lane < B) long_seq[2 * k + lane] = (uint32_t)(lane ? m >> 32 : m);
+            }
+        }
+        most = wave_scan(most, [](int x, int y) { return x > y ? x : y; });
         if (lane == 63) {
             pre[0] = 0;
-            pre[a.batch + 1] = most;
-        }
-        if (long_seq) {
-            const uint64_t m = __ballot(len > max_len);
-            if (lane < (a.batch + 31) / 32) long_seq[lane] = (uint32_t)(lane ? m >> 32 : m);
+            pre[B + 1] = most;
         }
         return;
     }
