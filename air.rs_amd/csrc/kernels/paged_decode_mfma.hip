@@ -264,6 +264,8 @@ constexpr int waves_per_simd(int dt) {
 constexpr int kernel_waves_per_simd(int dt, bool append) {
     return (append && dt == AIR_KV_FP8) ? 3 : waves_per_simd(dt);
 }
+// The workspace holds waves_per_simd's slices.
+static_assert(kernel_waves_per_simd(AIR_KV_FP8, true) <= waves_per_simd(AIR_KV_FP8), "the append's slices fit the workspace");
 
 // The build's waves per SIMD are its minimum and its maximum: with the
 // maximum the register allocator plans for that occupancy, not a higher one
