@@ -653,8 +653,8 @@ int plan_decode_f32(const air_kv_pool &p, int32_t n_q_heads, int32_t batch, int3
                     int32_t max_splits, DecodePlan *plan) {
     constexpr size_t kWsBytes = (size_t)24 << 20;
     const int nkv = p.desc.n_kv_heads, d = p.desc.head_dim, bs = p.desc.block_size;
-    const int64_t tiles_per_seq = ((int64_t)max_blocks * bs + 15) / 16;
-    if (tiles_per_seq > INT32_MAX) return fail(AIR_KV_E_INVALID_ARG, "max_blocks too large");
+    // lengths are 32-bit: a wider table's rest is never reached
+    const int64_t tiles_per_seq = std::min<int64_t>(((int64_t)max_blocks * bs + 15) / 16, ((int64_t)INT32_MAX + 15) / 16);
     int64_t nb = std::min<int64_t>(batch, kMaxBatch);
     nb = std::max<int64_t>(1, std::min<int64_t>(nb, INT32_MAX / std::max<int64_t>(tiles_per_seq, 1)));
     const int64_t per_slice = (int64_t)nkv * ((n_q_heads / nkv + kHeads - 1) / kHeads);
