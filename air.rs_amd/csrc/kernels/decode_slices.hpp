@@ -130,6 +130,10 @@ __device__ __forceinline__ void tile_prefix(const DecodeArgs &a, int bs, int32_t
             pre[0] = 0;
             pre[B + 1] = most;
         }
+        // lanes read what other lanes of their wave wrote: LDS serves a wave in
+        // order, this keeps the compiler from moving a read ahead of the writes
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         return;
     }
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
