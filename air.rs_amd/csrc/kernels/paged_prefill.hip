@@ -273,11 +273,6 @@ __device__ __forceinline__ void to_bf16x8_split(const Raw8<DT> &r, u32x4 &hi, u3
 // sequences or kRankItems items are taken slot by slot (slot slowest),
 // without ranking or splitting.
 
-struct PrefillSlot {
-    int b, kh, z, nz;
-    int p, ns, ord;            // piece, pieces of the slot (1: not split), split ordinal (-1: none)
-};
-
 // Keys the heaviest wave of slot z of a sequence needs (0: no work).
 __device__ __forceinline__ int64_t slot_keys(int64_t len, int64_t qlen, int G, int z) {
     if (qlen <= 0 || len < qlen) return 0;
@@ -686,8 +681,7 @@ void prefill_pipe_kernel(PrefillArgs a) {
     int32_t q0;
     int qlen;
     int64_t len;
-    if (!prefill_begin(a, b, kh, sl.z == 0 && sl.p == 0, D, q0, qlen, len)) return;
-    if (sl.z == 0 && sl.p == 0 && kh == 0) prefill_count_entries(a, b, BS, len);
+    if (!prefill_begin<BS, D>(a, sl, q0, qlen, len)) return;
     const int32_t *tbl = a.tables + (int64_t)b * a.max_blocks;
     const int q_offset = (int)(len - qlen);
     const int ntb = (qlen + kRows - 1) / kRows;

@@ -275,7 +275,7 @@ void prefill_f32_kernel(PrefillArgs a) {
     int32_t q0;
     int qlen;
     int64_t len;
-    if (!prefill_begin(a, b, kh, z == 0, d, q0, qlen, len)) return;
+    if (!prefill_begin<0, 0>(a, PrefillSlot{b, kh, z, 1, 0, 1, -1}, q0, qlen, len)) return;
     const int32_t *tbl = a.tables + (int64_t)b * a.max_blocks;
     const int bs_log2 = __builtin_ctz((unsigned)a.block_size), bs_mask = a.block_size - 1;
     const int sg_log2 = a.scale_group ? __builtin_ctz((unsigned)a.scale_group) : 0;
@@ -656,7 +656,13 @@ void prefill_f32_kernel(PrefillArgs a) {
         }
         __syncthreads();                                         // the next work group restages LDS
     }
-    if (z == 0 && kh == 0) prefill_count_entries(a, b, a.block_size, len);
+    // the out-of-pool table entries within the sequence's length, once per sequence
+    if (z == 0 && kh == 0) {
+        for (int64_t j = threadIdx.x; j < (len + a.block_size - 1) >> bs_log2; j += kThreads) {
+            const int32_t blk = tbl[j];
+            if (blk < 0 || blk >= a.num_blocks) atomicAdd(a.errors, 1ull);
+        }
+    }
 }
 
 template <int D, int PT, int NQ, int NK>

@@ -14,7 +14,7 @@ struct PrefillArgs {
     int32_t batch, max_blocks, total_q;
     int64_t max_len;               // max_blocks * block_size (set by launch_prefill)
     float scale_log2;              // softmax scale * log2(e)
-    int32_t n_kv_heads, group, scale_group, head_dim, block_size;
+    int32_t n_kv_heads, group, scale_group;
     int64_t num_blocks;
     const void *k_pages, *v_pages;
     const float *k_scales, *v_scales;
@@ -27,6 +27,7 @@ struct PrefillArgs {
     int32_t slots;                 // resident workgroups of the launch: the balance target
     void *ws;                      // key-split workspace (ns_max > 1)
     int32_t ws_units;              // split slots the workspace holds
+    int32_t head_dim, block_size;
     bool fp8;                      // launch_prefill_f32: 1-byte pages hold fp8 codes (else int8)
 };
 

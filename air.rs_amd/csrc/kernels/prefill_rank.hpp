@@ -31,41 +31,57 @@ __device__ __forceinline__ bool prefill_seq_ok(const PrefillArgs &a, int b) {
     return prefill_rows_ok(a, b) && len >= 0 && len <= a.max_len && qlen <= len;
 }
 
+// A workgroup's place in a launch.
+struct PrefillSlot {
+    int b, kh, z, nz;          // sequence, kv head, slot of it, slots per sequence
+    int p, ns, ord;            // piece, pieces of the slot (1: not split), split ordinal (-1: none)
+};
+
 // Per-(sequence, kv head) setup shared by the prefill kernels: reads the
-// sequence's rows and length, counts (once) an inconsistent sequence,
-// zero-fills its rows, and returns whether the workgroup has rows to compute.
-// Uniform per workgroup.  `first`: the sequence's first workgroup of this kv
-// head; d: the pool's head_dim.
-__device__ __forceinline__ bool prefill_begin(const PrefillArgs &a, int b, int kh, bool first, int d, int32_t &q0,
-                                              int &qlen, int64_t &len) {
-    const int tid = threadIdx.x;
-    const int G = a.group;
+// sequence's rows and length, counts (once) an inconsistent sequence and, with
+// BS > 0 (the block size), every out-of-pool table entry within its length
+// (else the caller counts them), zero-fills the rows of an inconsistent
+// sequence, and returns whether the workgroup has rows to compute.  Uniform
+// per workgroup.  D: the head_dim (0: the pool's, read from the arguments).
+// The table loop is written out here: as a function of its own it changed the
+// matrix-core kernel's register allocation (six int8 chunks of up to 512 tokens
+// over up to 6000, 64 heads over 8: 437.8 us, 435.3 this way).
+template <int BS, int D>
+__device__ bool prefill_begin(const PrefillArgs &a, const PrefillSlot &sl, int32_t &q0, int &qlen, int64_t &len) {
+    const int b = sl.b, kh = sl.kh, tid = threadIdx.x;
+    const int G = a.group, d = D ? D : a.head_dim;
     q0 = a.cu_q[b];
     len = a.lens[b];
     qlen = a.cu_q[b + 1] - q0;
-    if (prefill_seq_ok(a, b)) return qlen > 0;
-    if (first && kh == 0 && tid == 0) atomicAdd(a.errors, 1ull);
-    // rows of a sequence whose lengths are inconsistent become zeros
-    if (first && prefill_rows_ok(a, b)) {
-        const int64_t n = (int64_t)qlen * G * d;
-        for (int64_t i = tid; i < n; i += kRankThreads) {
-            const int64_t r = i / (G * d), e = i % (G * d);
-            const int64_t idx = ((int64_t)(q0 + r) * a.n_q_heads + kh * G) * d + e;
-            if (a.out_dtype == AIR_KV_F32) ((float *)a.out)[idx] = 0.0f;
-            else ((uint16_t *)a.out)[idx] = 0;
+    const bool rows_ok = prefill_rows_ok(a, b);
+    const bool seq_ok = prefill_seq_ok(a, b);
+    const int32_t *tbl = a.tables + (int64_t)b * a.max_blocks;
+    if (sl.z == 0 && sl.p == 0 && kh == 0) {
+        if (!seq_ok) {
+            if (tid == 0) atomicAdd(a.errors, 1ull);
+        } else if (qlen > 0) {
+            if constexpr (BS > 0) {
+                for (int64_t j = tid; j < (len + BS - 1) / BS; j += kRankThreads) {
+                    const int32_t blk = tbl[j];
+                    if (blk < 0 || blk >= a.num_blocks) atomicAdd(a.errors, 1ull);
+                }
+            }
         }
     }
-    return false;
-}
-
-// Counts the out-of-pool table entries within sequence b's length (once per
-// sequence that has query rows: one workgroup calls this).
-__device__ __forceinline__ void prefill_count_entries(const PrefillArgs &a, int b, int bs, int64_t len) {
-    const int32_t *tbl = a.tables + (int64_t)b * a.max_blocks;
-    for (int64_t j = threadIdx.x; j < (len + bs - 1) / bs; j += kRankThreads) {
-        const int32_t blk = tbl[j];
-        if (blk < 0 || blk >= a.num_blocks) atomicAdd(a.errors, 1ull);
+    if (!seq_ok) {
+        // rows of a sequence whose lengths are inconsistent become zeros
+        if (rows_ok && sl.z == 0 && sl.p == 0) {
+            const int64_t n = (int64_t)qlen * G * d;
+            for (int64_t i = tid; i < n; i += kRankThreads) {
+                const int64_t r = i / (G * d), e = i % (G * d);
+                const int64_t idx = ((int64_t)(q0 + r) * a.n_q_heads + kh * G) * d + e;
+                if (a.out_dtype == AIR_KV_F32) ((float *)a.out)[idx] = 0.0f;
+                else ((uint16_t *)a.out)[idx] = 0;
+            }
+        }
+        return false;
     }
+    return qlen > 0;
 }
 
 __device__ __forceinline__ int len_bucket(int64_t len) {   // 0 .. 248, monotone in len
