@@ -7,11 +7,11 @@
 #include <stdint.h>
 
 #include "decode_common.hpp"
+#include "decode_plan.hpp"
 
 namespace airkv {
 
 constexpr int kSliceThreads = 256;         // threads of every workgroup that calls these
-constexpr int kMaxBatch = 4096;            // sequences per launch (the host splits larger batches)
 
 // Reductions across the lanes 16 and 32 apart with the gfx950 lane-swap
 // instructions instead of LDS permutes.  permlane16_swap(v, v) returns
@@ -62,23 +62,6 @@ __device__ __forceinline__ void swap_lane_bit5(u32x4 &x0, u32x4 &x1) {
 
 __device__ __forceinline__ int64_t clamp_len(int64_t len, int64_t max_len) {
     return len < 0 ? 0 : (len > max_len ? max_len : len);
-}
-
-// Tiles per slice: an equal share of `total` over the resident waves, but at
-// least full_chunk once every SIMD has a wave (simd_slices per kv head), and
-// large enough that no sequence is cut into more than max_splits pieces.  A
-// sequence of T tiles starting anywhere meets at most ceil((T - 1) / chunk) +
-// 1 slices, so chunk >= ceil((T - 1) / (max_splits - 1)) for the longest
-// sequence (tmax tiles) bounds every one; max_splits 1 leaves one slice per
-// kv head.
-__device__ __forceinline__ int slice_chunk(int total, int slices, int simd_slices, int full_chunk,
-                                           int tmax, int max_splits) {
-    const int lone = (total + simd_slices - 1) / simd_slices;
-    int c = (total + slices - 1) / slices;
-    c = max(c, max(1, min(lone, full_chunk)));
-    if (max_splits <= 1) return c > total ? c : total;
-    const int cs = (tmax - 1 + max_splits - 2) / (max_splits - 1);
-    return c > cs ? c : cs;
 }
 
 // Inclusive sum / running maximum over a wave's lanes (DPP: row shifts, then

@@ -389,7 +389,7 @@ void decode_f32_kernel(DecodeArgs a) {
         const bool none = whole && !(l > 0.0f);  // no sum, every key at -inf: zeros, as the merge gives
         const float inv = whole ? 1.0f / l : 1.0f;
         const int64_t orow = ((int64_t)bq * a.n_q_heads + kh * G + g0 + r16) * d;
-        const int64_t prow = ((int64_t)kh * a.slots + bq + w) * G + g0 + r16;
+        const int64_t prow = ((int64_t)kh * a.slots + part_row(w, bq, s_pre[bq] >= lo)) * G + g0 + r16;
         unrolled<P::N>([&](auto pc) {
             constexpr int p = decltype(pc)::value, SZ = P::size(p);
 #pragma unroll
@@ -567,7 +567,6 @@ __global__ __launch_bounds__(kThreads) void decode_f32_merge_kernel(DecodeArgs a
         const int w0 = p0 / chunk, w1 = (p1 - 1) / chunk;
         if (w0 == w1) return;                            // written by its slice
         const int n = w1 - w0 + 1;
-        const int64_t row0 = ((int64_t)kh * a.slots + b + w0) * G + h;
         float m = -INFINITY, l = 0.0f;
         auto fold = [&](float pm, float pl, f32x4 pv) {
             if (pm == -INFINITY) return;
@@ -584,7 +583,8 @@ __global__ __launch_bounds__(kThreads) void decode_f32_merge_kernel(DecodeArgs a
 #pragma unroll
             for (int i = 0; i < kBatch; ++i) {
                 const int p = q + NG * i + grp;
-                const int64_t row = row0 + (int64_t)(p < n ? p : 0) * G;
+                const int w = w0 + (p < n ? p : 0);
+                const int64_t row = ((int64_t)kh * a.slots + part_row(w, b, w == w0)) * G + h;
                 pm[i] = p < n ? a.part_ml[row * 2] : -INFINITY;
                 pl[i] = a.part_ml[row * 2 + 1];
                 pv[i] = *reinterpret_cast<const f32x4 *>(a.part_o + row * d + (mine ? col : 0));
@@ -635,51 +635,31 @@ template <int D> int waves_of(int dtype, bool q_bf16) {
                                   : waves_per_simd<D, kBf16, false>();
 }
 
-size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
-
-size_t ws_size(int64_t n_q_heads, int64_t nb, int64_t slices, int64_t d) {
-    const size_t rows = (size_t)(n_q_heads * (slices + nb));
-    return align256((size_t)(nb + 2) * 4) + align256(rows * 2 * 4) + rows * d * 4;
-}
-
 }  // namespace
 
-// Slices per kv head and head chunk: one wave for every wave slot of the GPU,
-// at most batch * max_splits, and no more than keep the workspace within
-// kWsBytes or what one partial result per sequence and 256 tokens takes
-// (many query heads over few kv heads would otherwise ask for hundreds of
-// megabytes of partial results).
+static_assert(kWsBytes <= (size_t)AIR_KV_NOALLOC_SCRATCH_BYTES, "air_paged_decode_noalloc holds the plan's workspace");
+
 int plan_decode_f32(const air_kv_pool &p, int32_t n_q_heads, int32_t batch, int32_t max_blocks,
                     int32_t max_splits, DecodePlan *plan) {
-    constexpr size_t kWsBytes = (size_t)24 << 20;
-    const int nkv = p.desc.n_kv_heads, d = p.desc.head_dim, bs = p.desc.block_size;
-    // lengths are 32-bit: a wider table's rest is never reached
-    const int64_t tiles_per_seq = std::min<int64_t>(((int64_t)max_blocks * bs + 15) / 16, ((int64_t)INT32_MAX + 15) / 16);
-    int64_t nb = std::min<int64_t>(batch, kMaxBatch);
-    nb = std::max<int64_t>(1, std::min<int64_t>(nb, INT32_MAX / std::max<int64_t>(tiles_per_seq, 1)));
+    const int nkv = p.desc.n_kv_heads, d = p.desc.head_dim, dt = p.desc.dtype;
     const int64_t per_slice = (int64_t)nkv * ((n_q_heads / nkv + kHeads - 1) / kHeads);
-    auto slices_for = [&](bool q_bf16) {
-        const int dt = p.desc.dtype;
+    auto waves = [&](bool q_bf16) {
         const int wps = d <= 64    ? waves_of<64>(dt, q_bf16)
                         : d <= 96  ? waves_of<96>(dt, q_bf16)
                         : d <= 128 ? waves_of<128>(dt, q_bf16)
                                    : waves_of<256>(dt, q_bf16);
-        return std::min<int64_t>(((int64_t)p.cus * 4 * wps + per_slice - 1) / per_slice, nb * max_splits);
+        return (int64_t)p.cus * 4 * wps;
     };
-    const int64_t parts = std::max<int64_t>(1, std::min<int64_t>(max_splits, (tiles_per_seq + 15) / 16));
-    const size_t most = std::max(kWsBytes, (size_t)n_q_heads * nb * parts * (d + 2) * 4);
-    const int64_t fit = (int64_t)(most / ((size_t)n_q_heads * (d + 2) * 4)) - nb;
-    auto clamped = [&](int64_t n) { return (int32_t)std::max<int64_t>(1, std::min(n, fit)); };
-    // the bf16-query build runs at least as many waves: the workspace is its
-    const int32_t slices = clamped(slices_for(true));
+    const DecodeF32Plan pl = plan_f32(n_q_heads, per_slice, d, p.desc.block_size, batch, max_blocks, max_splits,
+                                      waves(true), waves(false));
     plan->mfma = false;
-    plan->dtype = p.desc.dtype;
-    plan->slices = slices;
-    plan->slices_qf32 = std::min(slices, clamped(slices_for(false)));
+    plan->dtype = dt;
+    plan->slices = (int32_t)pl.slices;
+    plan->slices_qf32 = (int32_t)pl.slices_qf32;
     plan->slices_append = 0;
-    plan->batch_per_launch = (int32_t)nb;
-    plan->slots = (int32_t)(slices + nb);
-    plan->ws_bytes = ws_size(n_q_heads, nb, slices, d);
+    plan->batch_per_launch = (int32_t)pl.batch;
+    plan->slots = (int32_t)pl.slots;
+    plan->ws_bytes = pl.ws_bytes;
     return AIR_KV_OK;
 }
 
@@ -703,9 +683,9 @@ hipError_t launch_decode_f32(const DecodeArgs &base, const DecodePlan &plan, voi
         char *ws = (char *)workspace;
         const size_t rows = (size_t)a.n_q_heads * plan.slots;
         a.prefix = (int32_t *)ws;
-        ws += align256((size_t)(plan.batch_per_launch + 2) * 4);
+        ws += decode_align256((size_t)(plan.batch_per_launch + 2) * 4);
         a.part_ml = (float *)ws;
-        ws += align256(rows * 2 * 4);
+        ws += decode_align256(rows * 2 * 4);
         a.part_o = (float *)ws;
         const hipError_t e = d <= 64    ? launch_d<64>(a, plan.dtype, s)
                              : d <= 96  ? launch_d<96>(a, plan.dtype, s)

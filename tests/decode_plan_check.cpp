@@ -1,0 +1,75 @@
+// Checks decode_plan.hpp against a walk over the pieces it describes: every cut
+// piece of a launch gets a row of its own inside the planned slots, the
+// workspace stays within its bound, and the plan uses the GPU's waves.
+// Prints "<cases> cases, <n> wrong".
+#include <algorithm>
+#include <cstdio>
+#include <random>
+#include <vector>
+
+#include "kernels/decode_plan.hpp"
+
+using namespace airkv;
+
+static long cases = 0, wrong = 0;
+static void check(bool ok, const char *what, long long a = 0, long long b = 0, long long c = 0) {
+    if (!ok && wrong++ < 20) std::printf("wrong: %s (%lld, %lld, %lld)\n", what, a, b, c);
+}
+
+// The pieces of sequences of these tiles in slices as the kernel cuts them.
+static void walk(const std::vector<int> &tiles, int slices, int simd, int full, int max_splits) {
+    ++cases;
+    long total = 0;
+    int tmax = 0;
+    for (int t : tiles) { total += t; tmax = std::max(tmax, t); }
+    if (!total) return;
+    const int chunk = slice_chunk((int)total, slices, simd, full, tmax, max_splits);
+    check(chunk >= 1 && (long)chunk * slices >= total, "the slices cover every tile", total, slices, chunk);
+    const long rows = part_rows(slices, (long)tiles.size());
+    long start = 0, last = -1;
+    for (int b = 0; b < (int)tiles.size(); start += tiles[b], ++b) {
+        if (!tiles[b]) continue;
+        const int w0 = (int)(start / chunk), w1 = (int)((start + tiles[b] - 1) / chunk);
+        check(w1 - w0 + 1 <= max_splits, "pieces per sequence", w1 - w0 + 1, max_splits);
+        if (w0 == w1) continue;
+        for (int w = w0; w <= w1; ++w) {
+            const int row = part_row(w, b, w == w0);
+            check(row > last && row < rows, "a row of its own inside the slots", row, last, rows);
+            check((w == w0) == (start >= (long)w * chunk), "the kernel's test of a first piece", w, w0);
+            last = row;
+        }
+    }
+}
+
+int main() {
+    std::mt19937 rng(5);
+    auto in = [&](int lo, int hi) { return lo + (int)(rng() % (unsigned)(hi - lo + 1)); };
+    for (int i = 0; i < 20000; ++i) {
+        const int B = i % 3 ? in(1, 40) : in(1, 1500), most = in(0, 3) ? in(1, 9) : in(1, 400);
+        std::vector<int> tiles(B);
+        for (int &t : tiles) t = in(0, most);
+        const int splits = in(0, 2) ? 64 : in(1, 256);
+        walk(tiles, in(1, std::min(4096, B * splits)), in(1, 1024), in(1, 4), splits);
+    }
+    // slices of a plan: waves of a 256-CU GPU, the cap or a row per (sequence, 256 tokens)
+    const size_t cap = kWsBytes;
+    for (int nkv : {1, 2, 4, 8, 16})
+        for (int group : {1, 4, 8, 16, 32, 71})
+            for (int d : {32, 64, 96, 128, 256})
+                for (int batch : {1, 4, 64, 253, 300, 380, 512, 1024, 2048, 4096, 5000})
+                    for (int blocks : {1, 4, 16, 64, 8192})
+                        for (int splits : {1, 2, 64, 256}) {
+                            ++cases;
+                            const int64_t nq = nkv * group, per = nkv * ((group + 15) / 16), row = nq * (d + 2) * 4;
+                            const DecodeF32Plan p = plan_f32(nq, per, d, 16, batch, blocks, splits, 4096, 3072);
+                            const int64_t parts = std::min<int64_t>(splits, (blocks + 15) / 16);
+                            check(p.ws_bytes <= std::max<size_t>(cap, (size_t)row * p.batch * parts), "workspace", (long long)p.ws_bytes, row, batch);
+                            check(p.slots == part_rows(p.slices, p.batch) && p.slices_qf32 <= p.slices && p.slices_qf32 >= 1, "slots");
+                            // half the partial rows of the cap at least, unless the waves or the splits are fewer
+                            const int64_t want = std::min(std::min<int64_t>((4096 + per - 1) / per, p.batch * splits),
+                                                          std::max<int64_t>(1, ((int64_t)cap - 20000) / row / 2));
+                            check(p.slices >= want, "slices of a wide batch", p.slices, want, batch);
+                        }
+    std::printf("%ld cases, %ld wrong\n", cases, wrong);
+    return wrong != 0;
+}

@@ -2,7 +2,8 @@
 groups, GQA groups above 16) against the oracle's gather + flash_decode, at the
 edges of its tiles: sequences around its 16-token tiles and the 64-tile windows
 of a slice, head_dim below each built size, groups around its 16 heads, batches
-on both sides of the 64 sequences one wave scans, and the step's appended row."""
+around the 64 sequences of a scan step and on both sides of the 256 a wave scans
+alone and of the 4096 of a launch, and the step's appended row."""
 import numpy as np
 import pytest
 
@@ -62,6 +63,26 @@ def test_decode_f32_append_rows(dtype, d, n_q, scale_group):
     q = np.random.default_rng(8).standard_normal((len(ctx), n_q, d)).astype(np.float32)
     q, got = _run_pair(cfg, pa, pb, host, tables, lens, k_new, v_new, q, q_f32=True)
     assert rel_err(got, host.paged_decode(q, tables, lens, chunk=64)) <= TOL_F32
+
+
+@pytest.mark.parametrize("dtype,d,n_kv,group,batch,bad", [
+    (airkv.F32, 64, 1, 2, 255, 254), (airkv.BF16, 64, 2, 4, 256, 70), (airkv.INT8, 96, 1, 2, 257, 256),
+    (airkv.BF16, 256, 2, 32, 400, 333), (airkv.F32, 32, 1, 1, 4100, 4098)])
+def test_decode_f32_wide_batches(dtype, d, n_kv, group, batch, bad):
+    """The step with batches on both sides of the 256 sequences one wave scans
+    and of the 4096 of a launch, and one whose partial rows fill the workspace's
+    bound; sequence `bad` is longer than its table: nothing is appended for it,
+    and it is counted."""
+    ctx = [(7 * i) % 61 for i in range(batch)]
+    cfg = workloads.Config("wide", n_kv * group, n_kv, d, 16, dtype, batch)
+    w, pa, pb, host, tables, lens, k_new, v_new = _setup(cfg, ctx, seed=21 + batch)
+    lens[bad] = tables.shape[1] * 16 + 5
+    mask = np.arange(batch) != bad
+    q = np.random.default_rng(9).standard_normal((batch, n_kv * group, d)).astype(np.float32)
+    q, got = _run_pair(cfg, pa, pb, host, tables, lens, k_new, v_new, q, q_f32=True, append_mask=mask)
+    want = host.paged_decode(q[mask], tables[mask], lens[mask], chunk=64)
+    assert rel_err(got[mask], want) <= TOL_F32
+    assert pa.error_count() > 0 and pb.error_count() > 0
 
 
 @pytest.mark.parametrize("d", [64, 96])
