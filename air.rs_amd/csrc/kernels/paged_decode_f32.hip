@@ -5,12 +5,14 @@
 // map takes any group, src/chunked_attn.rs:65-72).
 //
 // The work division is paged_decode_mfma.hip's: equal slices of the batch's
-// 16-token tiles, one wave each, merged by log-sum-exp
-// (src/flash_decode.rs:114-142).
+// 16-token tiles, merged by log-sum-exp (src/flash_decode.rs:114-142).  A slice
+// has one wave, or past 128 elements of head_dim the four of a workgroup, each
+// with a quarter of the columns; they add their shares of a tile's scores
+// through LDS.
 //
-// Per 16-token tile, with no LDS and no lane exchange: v_mfma_f32_16x16x4_f32
-// takes one element per lane and operand, and the contraction order is free,
-// so both operands come straight from wide page loads.
+// Per 16-token tile: v_mfma_f32_16x16x4_f32 takes one element per lane and
+// operand, and the contraction order is free, so both operands come straight
+// from wide page loads.
 //   S = K . Q^T   lane (row r16 = lane % 16, g4 = lane / 16) holds 8 elements
 //                 of token r16 per 32 of head_dim (key_elem below); product
 //                 (m, e) contracts the four lanes' e-th ones.  bf16 pages
@@ -185,18 +187,25 @@ __device__ __forceinline__ void store_out(const DecodeArgs &a, int64_t i, const 
     }
 }
 
-// Waves per SIMD an instantiation is built for and launched with.
-template <int D, int PT, bool QB> constexpr int waves_per_simd() {
-    return PT == kF32 ? (D <= 64 ? 3 : D <= 128 ? 2 : 1)
-           : QB       ? (D <= 96 ? 4 : D <= 128 ? 3 : 2)
-           : D <= 64  ? (PT == kBf16 ? 4 : 3)
-           : D <= 96  ? 3
-           : D <= 128 ? (PT == kBf16 ? 3 : 2)
-                      : 1;
+// A workgroup barrier that orders LDS only (page loads stay in flight).
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// QB: bf16 queries over bf16 pages (else the queries enter as f32).
-template <int D, int PT, bool QB>
+// Waves per SIMD an instantiation is built for and launched with.
+template <int D, int PT, bool QB> constexpr int waves_per_simd() {
+    return PT == kF32 ? (D <= 64 ? 3 : 2)
+           : QB       ? (D <= 96 ? 4 : 3)
+           : D <= 64  ? (PT == kBf16 ? 4 : 3)
+           : D <= 96  ? 3
+                      : (PT == kBf16 ? 3 : 2);
+}
+
+// D: a wave's columns.  QB: bf16 queries over bf16 pages (else the queries enter
+// as f32).  TEAM: the workgroup's waves share a slice, D columns of head_dim each.
+template <int D, int PT, bool QB, bool TEAM>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(waves_per_simd<D, PT, QB>(), waves_per_simd<D, PT, QB>())))
 void decode_f32_kernel(DecodeArgs a) {
     static_assert(!QB || PT == kBf16, "bf16 products take bf16 pages");
@@ -213,13 +222,15 @@ void decode_f32_kernel(DecodeArgs a) {
         for (int i = threadIdx.x; i <= B; i += kThreads) a.prefix[i] = s_pre[i];
         if (threadIdx.x == 0) a.prefix[B + 1] = chunk;
     }
+    __shared__ f32x4 s_part[TEAM ? 2 : 1][TEAM ? kWaves : 1][TEAM ? 64 : 1];   // a tile's scores by wave
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g4 = lane >> 4, r16 = lane & 15;
     const int G = a.group, d = a.head_dim;
-    // Consecutive waves take consecutive kv heads of one slice (neighbouring
-    // pages), then the slice's other head chunks.
-    const int gw = blockIdx.x * kWaves + wave;
+    const int col0 = TEAM ? D * wave : 0, dw = d - col0;        // the wave's columns: the first D of dw (none: dw <= 0)
+    // Consecutive waves (or teams) take consecutive kv heads of one slice
+    // (neighbouring pages), then the slice's other head chunks.
+    const int gw = TEAM ? (int)blockIdx.x : blockIdx.x * kWaves + wave;
     const int chunks = (G + kHeads - 1) / kHeads;
     const int kh = gw % a.n_kv_heads, rest = gw / a.n_kv_heads;
     const int hc = rest % chunks, w = rest / chunks;
@@ -254,7 +265,7 @@ void decode_f32_kernel(DecodeArgs a) {
 
     // The lane's elements of 32: 8 g4 .. + 8, or for f32 pages read by lines, as
     // their two 16-byte loads come, 4 g4 .. + 4 and 16 + 4 g4 .. + 4.
-    auto key_elem = [&](int half) { return PT == kF32 && D < 256 ? 16 * half + 4 * g4 : 8 * g4 + 4 * half; };
+    auto key_elem = [&](int half) { return PT == kF32 ? 16 * half + 4 * g4 : 8 * g4 + 4 * half; };
     // ---- queries (head r16), the same elements; heads past the chunk and
     // columns past head_dim read zeros outside the descriptor
     u32x4 qb[QB ? KM : 1];
@@ -265,13 +276,13 @@ void decode_f32_kernel(DecodeArgs a) {
         const __amdgpu_buffer_rsrc_t rq = rsrc((const char *)a.q + row * d * qbytes, gn * d * qbytes);
 #pragma unroll
         for (int m = 0; m < KM; ++m) {
-            const int off = (r16 * d + 32 * m) * qbytes;
+            const int off = (r16 * d + col0 + 32 * m) * qbytes;
             if constexpr (QB) {
-                qb[m] = __builtin_amdgcn_raw_buffer_load_b128(rq, 32 * m < d ? off + 16 * g4 : kOutside, 0, 0);
+                qb[m] = __builtin_amdgcn_raw_buffer_load_b128(rq, 32 * m < dw ? off + 16 * g4 : kOutside, 0, 0);
             } else {
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {
-                    const int at = 32 * m < d ? off + key_elem(half) * qbytes : kOutside;
+                    const int at = 32 * m < dw ? off + key_elem(half) * qbytes : kOutside;
                     uint32_t x[4];
                     if (a.q_dtype == AIR_KV_F32) {
                         load_words<16, 0>(rq, at, 0, x);
@@ -292,12 +303,11 @@ void decode_f32_kernel(DecodeArgs a) {
     // 4 g4 (step i adds i rows), and their scales.
     // Whole-line key loads: load h of a 128-byte line column reads, in lane
     // l, row 8 h + l % 8, 16 bytes at 64 bit3(l) + 32 bit5(l) + 16 bit4(l).
-    // (f32 rows of 256 are left out: the transposes' registers cost more.)
-    constexpr bool LINES = !kByte<PT> && D * EB % 128 == 0 && D * EB < 1024;
+    constexpr bool LINES = !kByte<PT> && D * EB % 128 == 0;
     const bool lines = LINES && d * EB % 128 == 0;
-    const int k_off = lines ? (lane & 7) * d * EB + 64 * ((lane >> 3) & 1) + 32 * (lane >> 5) + 16 * ((lane >> 4) & 1)
-                            : (r16 * d + 8 * g4) * EB;
-    const int v_off = 4 * g4 * d * EB;
+    const int k_off = col0 * EB + (lines ? (lane & 7) * d * EB + 64 * ((lane >> 3) & 1) + 32 * (lane >> 5) + 16 * ((lane >> 4) & 1)
+                                         : (r16 * d + 8 * g4) * EB);
+    const int v_off = (4 * g4 * d + col0) * EB;
     uint32_t kw[KM][8 * EB / 4], vw[4][P::N][P::kMost * EB / 4 > 0 ? P::kMost * EB / 4 : 1];
     float ksc[kByte<PT> ? KM : 1], vsc[kByte<PT> ? 4 : 1][kByte<PT> ? P::N : 1];
 
@@ -307,7 +317,7 @@ void decode_f32_kernel(DecodeArgs a) {
         for (int i = 0; i < 4; ++i)
             unrolled<P::N>([&](auto pc) {
                 constexpr int p = decltype(pc)::value, SZ = P::size(p), base = 16 * P::first(p);
-                const int voff = base + SZ * r16 < d ? v_off + SZ * r16 * EB : kOutside;
+                const int voff = base + SZ * r16 < dw ? v_off + SZ * r16 * EB : kOutside;
                 load_words<SZ * EB, kValueAux>(rv, voff, (i * d + base) * EB, vw[i][p]);
             });
         if constexpr (kByte<PT>) {
@@ -317,7 +327,7 @@ void decode_f32_kernel(DecodeArgs a) {
                     constexpr int p = decltype(pc)::value;
                     const int at = 16 * P::first(p) + P::size(p) * r16;
                     vsc[i][p] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                        rvs, at < d ? (4 * g4 * n_sc + (at >> sg_log2)) * 4 : kOutside, i * n_sc * 4, 0));
+                        rvs, at < dw ? (4 * g4 * n_sc + ((col0 + at) >> sg_log2)) * 4 : kOutside, i * n_sc * 4, 0));
                 });
         }
     };
@@ -330,8 +340,8 @@ void decode_f32_kernel(DecodeArgs a) {
         if (ok && ((new_m >> idx) & 1)) {
             // the step's new token: row nv - 1 of this tile, lanes 0 .. d/8 - 1
             // its key, the next d/8 its value; in the page before the tile
-            // loads (the waves of a group's head chunks each write the same
-            // bytes, so none depends on another's)
+            // loads (the waves of a team and of a group's head chunks each write
+            // the same bytes, so none depends on another's)
             const int bq = __builtin_amdgcn_readlane(seq_l, idx);
             const int64_t row = row0 + __builtin_amdgcn_readlane(nv_l, idx) - 1;
             const int per = d >> 3, c = lane < per ? lane : lane - per;
@@ -360,12 +370,12 @@ void decode_f32_kernel(DecodeArgs a) {
             for (int c = 0; c < KM * 8 * EB / 32; ++c)
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
-                    load_words<16, kLineAux>(rk, 128 * c < d * EB ? k_off : kOutside, 128 * c + 8 * h * d * EB,
+                    load_words<16, kLineAux>(rk, 128 * c < dw * EB ? k_off : kOutside, 128 * c + 8 * h * d * EB,
                                              &kw[0][0] + 8 * c + 4 * h);
         } else {
 #pragma unroll
             for (int m = 0; m < KM; ++m) {
-                load_words<8 * EB, kKeyAux>(rk, 32 * m < d ? k_off : kOutside, 32 * m * EB, kw[m]);
+                load_words<8 * EB, kKeyAux>(rk, 32 * m < dw ? k_off : kOutside, 32 * m * EB, kw[m]);
             }
         }
         if constexpr (kByte<PT>) {
@@ -374,7 +384,7 @@ void decode_f32_kernel(DecodeArgs a) {
 #pragma unroll
             for (int m = 0; m < KM; ++m)
                 ksc[m] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                    rks, 32 * m < d ? (r16 * n_sc + ((32 * m + 8 * g4) >> sg_log2)) * 4 : kOutside, 0, 0));
+                    rks, 32 * m < dw ? (r16 * n_sc + ((col0 + 32 * m + 8 * g4) >> sg_log2)) * 4 : kOutside, 0, 0));
         }
         load_values();
         return ok;
@@ -388,14 +398,14 @@ void decode_f32_kernel(DecodeArgs a) {
         const bool whole = w0 == w1;             // the whole sequence: final output
         const bool none = whole && !(l > 0.0f);  // no sum, every key at -inf: zeros, as the merge gives
         const float inv = whole ? 1.0f / l : 1.0f;
-        const int64_t orow = ((int64_t)bq * a.n_q_heads + kh * G + g0 + r16) * d;
+        const int64_t orow = ((int64_t)bq * a.n_q_heads + kh * G + g0 + r16) * d + col0;
         const int64_t prow = ((int64_t)kh * a.slots + part_row(w, bq, s_pre[bq] >= lo)) * G + g0 + r16;
         unrolled<P::N>([&](auto pc) {
             constexpr int p = decltype(pc)::value, SZ = P::size(p);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int at = 16 * P::first(p) + SZ * (4 * g4 + i);
-                if (at >= d) continue;
+                if (at >= dw) continue;
                 float v[SZ];
 #pragma unroll
                 for (int j = 0; j < SZ; ++j) v[j] = none ? 0.0f : acc[p][j][i] * inv;
@@ -404,11 +414,11 @@ void decode_f32_kernel(DecodeArgs a) {
                 } else {
 #pragma unroll
                     for (int j = 0; j < SZ; j += 2)
-                        *reinterpret_cast<f32x2 *>(a.part_o + prow * d + at + j) = f32x2{v[j], v[j + 1]};
+                        *reinterpret_cast<f32x2 *>(a.part_o + prow * d + col0 + at + j) = f32x2{v[j], v[j + 1]};
                 }
             }
         });
-        if (!whole && g4 == 0) {
+        if (!whole && g4 == 0 && col0 == 0) {
             a.part_ml[prow * 2] = m_run;
             a.part_ml[prow * 2 + 1] = l;
         }
@@ -427,7 +437,7 @@ void decode_f32_kernel(DecodeArgs a) {
                 for (int j = 0; j < P::kMost; ++j) acc[p][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         }
         // a table entry outside the pool is counted and its tile masked out
-        if (!ok && lane == 0 && hc == 0) atomicAdd(a.errors, 1ull);
+        if (!ok && lane == 0 && hc == 0 && col0 == 0) atomicAdd(a.errors, 1ull);
         const int nv = ok ? __builtin_amdgcn_readlane(nv_l, idx) : 0;
         if constexpr (LINES) {
             if (lines) {
@@ -468,7 +478,17 @@ void decode_f32_kernel(DecodeArgs a) {
         for (int st = 1; st < KM; st <<= 1)
 #pragma unroll
             for (int m = 0; m + st < KM; m += 2 * st) part[m] += part[m + st];
-        const f32x4 s = part[0];
+        f32x4 s = part[0];
+        if constexpr (TEAM) {
+            // the columns' shares, added in one order by every wave.  Two
+            // buffers, one barrier a tile: a wave writes a buffer again only
+            // past the barrier of the tile between, which it reached after
+            // reading this one, as all of them did.
+            f32x4 (*sp)[64] = s_part[k & 1];
+            sp[wave][lane] = s;
+            lds_barrier();
+            s = (sp[0][lane] + sp[1][lane]) + (sp[2][lane] + sp[3][lane]);
+        }
         float sc[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) sc[i] = s[i] * a.scale_log2;
@@ -604,28 +624,36 @@ __global__ __launch_bounds__(kThreads) void decode_f32_merge_kernel(DecodeArgs a
     if (grp == 0 && mine) store_out<4>(a, oi, o);
 }
 
-template <int D, int PT, bool QB>
+template <int D, int PT, bool QB, bool TEAM>
 hipError_t launch_one(const DecodeArgs &a, hipStream_t s) {
     const int chunks = (a.group + kHeads - 1) / kHeads;
-    const int64_t waves = (int64_t)a.n_kv_heads * chunks * a.slices;
-    hipLaunchKernelGGL((decode_f32_kernel<D, PT, QB>), dim3((unsigned)((waves + kWaves - 1) / kWaves)),
-                       dim3(kThreads), 0, s, a);
+    const int64_t units = (int64_t)a.n_kv_heads * chunks * a.slices, per = TEAM ? 1 : kWaves;
+    hipLaunchKernelGGL((decode_f32_kernel<D, PT, QB, TEAM>), dim3((unsigned)((units + per - 1) / per)), dim3(kThreads),
+                       0, s, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const dim3 grid((unsigned)a.batch, (unsigned)a.n_kv_heads, (unsigned)((a.group + kWaves - 1) / kWaves));
-    if constexpr (D <= 64) hipLaunchKernelGGL(decode_f32_merge_kernel<64>, grid, dim3(kThreads), 0, s, a);
-    else if constexpr (D <= 128) hipLaunchKernelGGL(decode_f32_merge_kernel<128>, grid, dim3(kThreads), 0, s, a);
-    else hipLaunchKernelGGL(decode_f32_merge_kernel<256>, grid, dim3(kThreads), 0, s, a);
+    if constexpr (TEAM) hipLaunchKernelGGL(decode_f32_merge_kernel<256>, grid, dim3(kThreads), 0, s, a);
+    else if constexpr (D <= 64) hipLaunchKernelGGL(decode_f32_merge_kernel<64>, grid, dim3(kThreads), 0, s, a);
+    else hipLaunchKernelGGL(decode_f32_merge_kernel<128>, grid, dim3(kThreads), 0, s, a);
     return hipGetLastError();
 }
 
-template <int D>
+template <int D, bool TEAM>
 hipError_t launch_d(const DecodeArgs &a, int dtype, hipStream_t s) {
-    if (dtype == AIR_KV_F32) return launch_one<D, kF32, false>(a, s);
-    if (dtype == AIR_KV_INT8) return launch_one<D, kInt8, false>(a, s);
-    if (dtype == AIR_KV_FP8) return launch_one<D, kFp8, false>(a, s);
-    return a.q_dtype == AIR_KV_BF16 ? launch_one<D, kBf16, true>(a, s) : launch_one<D, kBf16, false>(a, s);
+    if (dtype == AIR_KV_F32) return launch_one<D, kF32, false, TEAM>(a, s);
+    if (dtype == AIR_KV_INT8) return launch_one<D, kInt8, false, TEAM>(a, s);
+    if (dtype == AIR_KV_FP8) return launch_one<D, kFp8, false, TEAM>(a, s);
+    return a.q_dtype == AIR_KV_BF16 ? launch_one<D, kBf16, true, TEAM>(a, s) : launch_one<D, kBf16, false, TEAM>(a, s);
 }
+
+// Past 128 elements a wave that holds a whole tile runs alone on its SIMD with
+// nothing to overlap, so a workgroup's four waves share the tile, 64 columns
+// each (88 sequences of 114 tokens, 8 heads over 4, f32 pages of 256: 25.9 us, 37.2
+// with a wave alone, 30.0 on the vector kernel before it).  Two waves of 96 columns
+// for up to 192 elements were 2 to 10% slower.
+constexpr int kTeamColumns = 64;
+bool team(int d) { return d > 128; }
 
 template <int D> int waves_of(int dtype, bool q_bf16) {
     return dtype == AIR_KV_F32    ? waves_per_simd<D, kF32, false>()
@@ -646,9 +674,9 @@ int plan_decode_f32(const air_kv_pool &p, int32_t n_q_heads, int32_t batch, int3
     auto waves = [&](bool q_bf16) {
         const int wps = d <= 64    ? waves_of<64>(dt, q_bf16)
                         : d <= 96  ? waves_of<96>(dt, q_bf16)
-                        : d <= 128 ? waves_of<128>(dt, q_bf16)
-                                   : waves_of<256>(dt, q_bf16);
-        return (int64_t)p.cus * 4 * wps;
+                        : !team(d) ? waves_of<128>(dt, q_bf16)
+                                   : waves_of<kTeamColumns>(dt, q_bf16);
+        return (int64_t)p.cus * (team(d) ? 1 : 4) * wps;
     };
     const DecodeF32Plan pl = plan_f32(n_q_heads, per_slice, d, p.desc.block_size, batch, max_blocks, max_splits,
                                       waves(true), waves(false));
@@ -687,10 +715,10 @@ hipError_t launch_decode_f32(const DecodeArgs &base, const DecodePlan &plan, voi
         a.part_ml = (float *)ws;
         ws += decode_align256(rows * 2 * 4);
         a.part_o = (float *)ws;
-        const hipError_t e = d <= 64    ? launch_d<64>(a, plan.dtype, s)
-                             : d <= 96  ? launch_d<96>(a, plan.dtype, s)
-                             : d <= 128 ? launch_d<128>(a, plan.dtype, s)
-                                        : launch_d<256>(a, plan.dtype, s);
+        const hipError_t e = d <= 64    ? launch_d<64, false>(a, plan.dtype, s)
+                             : d <= 96  ? launch_d<96, false>(a, plan.dtype, s)
+                             : !team(d) ? launch_d<128, false>(a, plan.dtype, s)
+                                        : launch_d<kTeamColumns, true>(a, plan.dtype, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

@@ -28,7 +28,7 @@ CASES = [(dt, d, 2, 4, 16, 32, 15) for dt in (airkv.F32, airkv.BF16, airkv.INT8,
          for d in (32, 64, 96, 160, 256)] + [
     (airkv.F32, 128, 8, 1, 32, 32, 15), (airkv.F32, 128, 1, 17, 16, 32, 15), (airkv.BF16, 128, 1, 40, 32, 32, 15),
     (airkv.INT8, 128, 2, 7, 16, 16, 15), (airkv.FP8, 64, 2, 16, 32, 8, 15), (airkv.BF16, 224, 2, 16, 32, 32, 15),
-    (airkv.BF16, 64, 8, 4, 16, 32, 65), (airkv.F32, 64, 4, 2, 16, 32, 130), (airkv.INT8, 96, 1, 3, 32, 32, 64),
+    (airkv.F32, 192, 1, 3, 16, 32, 15), (airkv.FP8, 192, 2, 4, 32, 64, 15), (airkv.BF16, 64, 8, 4, 16, 32, 65), (airkv.F32, 64, 4, 2, 16, 32, 130), (airkv.INT8, 96, 1, 3, 32, 32, 64),
 ]
 
 
