@@ -18,7 +18,8 @@ struct DecodeArgs {
     int32_t batch, max_blocks;
     int32_t slices, slots;         // balanced slices per kv head, partial rows per (kv head, query head)
     int32_t simd_slices;           // slices per kv head that give every SIMD one wave
-    int32_t max_splits;            // pieces per sequence at most
+    int32_t max_splits;            // partitions of a sequence at most
+    int32_t seq_pieces;            // f32-precision kernel: slices of each sequence's own (0: of the batch's tiles)
     float scale_log2;              // softmax scale * log2(e): exp(x*s) == exp2(x*scale_log2)
     int32_t n_kv_heads, block_size, scale_group, group, head_dim;
     int64_t num_blocks;

@@ -44,6 +44,7 @@ hipError_t launch_decode(const air_kv_pool &p, hipStream_t s, const DecodePlan &
     const int waves = p.desc.n_kv_heads * ((plan.group + 15) / 16);   // per slice
     a.simd_slices = (4 * p.cus + waves - 1) / waves;
     a.slices = plan.slices; a.slots = plan.slots; a.max_splits = plan.max_splits;
+    a.seq_pieces = plan.seq_pieces;
     a.scale_log2 = scale * 1.4426950408889634f;
     a.n_kv_heads = p.desc.n_kv_heads; a.block_size = p.desc.block_size;
     a.scale_group = p.desc.scale_group; a.group = plan.group; a.num_blocks = p.desc.num_blocks;

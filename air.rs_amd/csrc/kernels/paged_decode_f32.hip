@@ -63,11 +63,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = kSliceThreads;
 constexpr int kWaves = kThreads / 64;
-// Tiles per slice at least once every SIMD has a wave: these waves' products
-// keep a SIMD less busy than the loads they wait for (64 sequences of 16 to 300
-// tokens, bf16 pages of 64: 13.8 us at one tile, 15.0 at four; 16 of 100 to 800,
-// f32 pages, 14.0 and 15.2).
-constexpr int kFullChunk = 1;
 constexpr int kHeads = 16;                 // query heads of a kv head per wave
 constexpr int kBufferWord3 = 0x00020000;   // raw buffer access
 constexpr int kOutside = 1 << 30;          // a lane offset no page tile reaches: reads as zero
@@ -217,7 +212,7 @@ void decode_f32_kernel(DecodeArgs a) {
     tile_prefix(a, a.block_size, s_pre, s_wsum, s_long);
     const int B = a.batch;
     const int total = s_pre[B];
-    const int chunk = slice_chunk(total, a.slices, a.simd_slices, kFullChunk, s_pre[B + 1], a.max_splits);
+    const int chunk = a.seq_pieces ? 0 : shared_chunk(total, a.slices, a.simd_slices, s_pre[B + 1], a.max_splits);
     if (blockIdx.x == 0) {                     // for the merge kernel: prefix, then the chunk
         for (int i = threadIdx.x; i <= B; i += kThreads) a.prefix[i] = s_pre[i];
         if (threadIdx.x == 0) a.prefix[B + 1] = chunk;
@@ -234,10 +229,22 @@ void decode_f32_kernel(DecodeArgs a) {
     const int chunks = (G + kHeads - 1) / kHeads;
     const int kh = gw % a.n_kv_heads, rest = gw / a.n_kv_heads;
     const int hc = rest % chunks, w = rest / chunks;
-    if (w >= a.slices || (int64_t)w * chunk >= total) return;
+    int lo, hi;                                // the slice's tiles
+    if (a.seq_pieces) {
+        const int b = w / a.seq_pieces;
+        if (b >= B) return;
+        const int step = piece_tiles(s_pre[b + 1] - s_pre[b], a.seq_pieces);
+        lo = s_pre[b] + w % a.seq_pieces * step;
+        hi = s_pre[b + 1] - lo < step ? s_pre[b + 1] : lo + step;
+        if (lo >= hi) return;
+    } else {
+        if (w >= a.slices || (int64_t)w * chunk >= total) return;
+        lo = w * chunk;
+        hi = total - lo < chunk ? total : lo + chunk;
+    }
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    hi = __builtin_amdgcn_readfirstlane(hi);
     const int g0 = hc * kHeads, gn = G - g0 < kHeads ? G - g0 : kHeads;   // this wave's heads of the group
-    const int lo = w * chunk;
-    const int hi = total - lo < chunk ? total : lo + chunk;
     const int64_t max_len = (int64_t)a.max_blocks * a.block_size;
     const int bs_log2 = __builtin_ctz((unsigned)a.block_size);
     const int sg_log2 = kByte<PT> ? __builtin_ctz((unsigned)a.scale_group) : 0;
@@ -393,13 +400,13 @@ void decode_f32_kernel(DecodeArgs a) {
     // The piece of sequence bq held by this wave ends: write it out.
     auto emit = [&](int bq) __attribute__((always_inline)) {
         const float l = sum_x32(sum_x16(l_run));
-        const int w0 = s_pre[bq] / chunk, w1 = (s_pre[bq + 1] - 1) / chunk;
+        const bool starts = s_pre[bq] >= lo;
         if (r16 >= gn) return;
-        const bool whole = w0 == w1;             // the whole sequence: final output
+        const bool whole = starts && s_pre[bq + 1] <= hi;   // the whole sequence: final output
         const bool none = whole && !(l > 0.0f);  // no sum, every key at -inf: zeros, as the merge gives
         const float inv = whole ? 1.0f / l : 1.0f;
         const int64_t orow = ((int64_t)bq * a.n_q_heads + kh * G + g0 + r16) * d + col0;
-        const int64_t prow = ((int64_t)kh * a.slots + part_row(w, bq, s_pre[bq] >= lo)) * G + g0 + r16;
+        const int64_t prow = ((int64_t)kh * a.slots + (a.seq_pieces ? w : part_row(w, bq, starts))) * G + g0 + r16;
         unrolled<P::N>([&](auto pc) {
             constexpr int p = decltype(pc)::value, SZ = P::size(p);
 #pragma unroll
@@ -584,9 +591,10 @@ __global__ __launch_bounds__(kThreads) void decode_f32_merge_kernel(DecodeArgs a
     const int64_t oi = ((int64_t)b * a.n_q_heads + kh * G + h) * d + col;
     float o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (p0 != p1) {
-        const int w0 = p0 / chunk, w1 = (p1 - 1) / chunk;
-        if (w0 == w1) return;                            // written by its slice
-        const int n = w1 - w0 + 1;
+        const int step = a.seq_pieces ? piece_tiles(p1 - p0, a.seq_pieces) : chunk;
+        const int w0 = a.seq_pieces ? 0 : p0 / step;
+        const int n = a.seq_pieces ? (p1 - p0 + step - 1) / step : (p1 - 1) / step - w0 + 1;
+        if (n == 1) return;                              // written by its slice
         float m = -INFINITY, l = 0.0f;
         auto fold = [&](float pm, float pl, f32x4 pv) {
             if (pm == -INFINITY) return;
@@ -604,7 +612,8 @@ __global__ __launch_bounds__(kThreads) void decode_f32_merge_kernel(DecodeArgs a
             for (int i = 0; i < kBatch; ++i) {
                 const int p = q + NG * i + grp;
                 const int w = w0 + (p < n ? p : 0);
-                const int64_t row = ((int64_t)kh * a.slots + part_row(w, b, w == w0)) * G + h;
+                const int64_t row =
+                    ((int64_t)kh * a.slots + (a.seq_pieces ? b * a.seq_pieces + w : part_row(w, b, w == w0))) * G + h;
                 pm[i] = p < n ? a.part_ml[row * 2] : -INFINITY;
                 pl[i] = a.part_ml[row * 2 + 1];
                 pv[i] = *reinterpret_cast<const f32x4 *>(a.part_o + row * d + (mine ? col : 0));
@@ -685,6 +694,7 @@ int plan_decode_f32(const air_kv_pool &p, int32_t n_q_heads, int32_t batch, int3
     plan->slices = (int32_t)pl.slices;
     plan->slices_qf32 = (int32_t)pl.slices_qf32;
     plan->slices_append = 0;
+    plan->seq_pieces = (int32_t)pl.seq_pieces;
     plan->batch_per_launch = (int32_t)pl.batch;
     plan->slots = (int32_t)pl.slots;
     plan->ws_bytes = pl.ws_bytes;
@@ -698,6 +708,7 @@ hipError_t launch_decode_f32(const DecodeArgs &base, const DecodePlan &plan, voi
         a.batch = std::min(base.batch - b0, plan.batch_per_launch);
         a.slices = base.q_dtype == AIR_KV_F32 ? plan.slices_qf32 : plan.slices;
         a.slots = plan.slots;
+        a.simd_slices = team(d) ? (base.simd_slices + kWaves - 1) / kWaves : base.simd_slices;
         const int64_t q_row = (int64_t)b0 * a.n_q_heads * d;
         a.q = (const char *)base.q + q_row * (base.q_dtype == AIR_KV_F32 ? 4 : 2);
         a.out = (char *)base.out + q_row * (base.out_dtype == AIR_KV_F32 ? 4 : 2);

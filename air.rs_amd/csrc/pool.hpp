@@ -40,8 +40,9 @@ struct DecodePlan {
     int32_t slices_qf32;  // the same for f32 queries (their kernel may hold fewer waves per SIMD)
     int32_t slices_append;  // the same for the fused append + decode
     int32_t batch_per_launch;
-    int32_t max_splits;   // pieces per sequence at most
-    int32_t slots;        // partial rows per (kv head, q head of the group): slices + batch
+    int32_t max_splits;   // partitions of a sequence at most
+    int32_t seq_pieces;   // slices of each sequence's own (0: of the batch's tiles)
+    int32_t slots;        // partial rows per (kv head, q head of the group)
     size_t ws_bytes;
 };
 int plan_decode(const air_kv_pool &pool, int32_t n_q_heads, int32_t batch, int32_t max_blocks,

@@ -262,7 +262,9 @@ int air_paged_decode_workspace_size(const air_kv_pool *pool, int32_t n_q_heads, 
  * with scale_group >= 32 -- take a kernel with 16-bit operands; other pools
  * (F32 pages, other head dims, groups above 16, small scale groups) one that
  * keeps queries, keys, probabilities and values at f32 precision, 16 query
- * heads of a kv head to a wave.  Out-of-pool table
+ * heads of a kv head to a wave; there up to four slices share a partition where
+ * max_splits leaves the GPU idle, and max_splits 1 gives each sequence slices of
+ * its own, so that its result does not depend on the others'.  Out-of-pool table
  * entries are skipped and counted (air_kv_pool_error_count); seq_lens outside
  * [0, max_blocks * block_size] are clamped and counted.  A sequence of length
  * 0 produces zeros.  The workspace is device

@@ -16,21 +16,23 @@ static void check(bool ok, const char *what, long long a = 0, long long b = 0, l
     if (!ok && wrong++ < 20) std::printf("wrong: %s (%lld, %lld, %lld)\n", what, a, b, c);
 }
 
-// The pieces of sequences of these tiles in slices as the kernel cuts them.
+// The pieces of sequences of these tiles in slices as the kernels cut them (full
+// 0: the f32-precision one).
 static void walk(const std::vector<int> &tiles, int slices, int simd, int full, int max_splits) {
     ++cases;
     long total = 0;
     int tmax = 0;
     for (int t : tiles) { total += t; tmax = std::max(tmax, t); }
     if (!total) return;
-    const int chunk = slice_chunk((int)total, slices, simd, full, tmax, max_splits);
+    const int chunk = full ? slice_chunk((int)total, slices, simd, full, tmax, max_splits)
+                           : shared_chunk((int)total, slices, simd, tmax, max_splits);
     check(chunk >= 1 && (long)chunk * slices >= total, "the slices cover every tile", total, slices, chunk);
     const long rows = part_rows(slices, (long)tiles.size());
     long start = 0, last = -1;
     for (int b = 0; b < (int)tiles.size(); start += tiles[b], ++b) {
         if (!tiles[b]) continue;
         const int w0 = (int)(start / chunk), w1 = (int)((start + tiles[b] - 1) / chunk);
-        check(w1 - w0 + 1 <= max_splits, "pieces per sequence", w1 - w0 + 1, max_splits);
+        check(w1 - w0 + 1 <= max_splits * (full ? 1 : kSharing), "pieces per sequence", w1 - w0 + 1, max_splits);
         if (w0 == w1) continue;
         for (int w = w0; w <= w1; ++w) {
             const int row = part_row(w, b, w == w0);
@@ -38,6 +40,16 @@ static void walk(const std::vector<int> &tiles, int slices, int simd, int full, 
             check((w == w0) == (start >= (long)w * chunk), "the kernel's test of a first piece", w, w0);
             last = row;
         }
+    }
+}
+
+// The same where every sequence has `pieces` slices of its own.
+static void walk_own(const std::vector<int> &tiles, int pieces) {
+    ++cases;
+    for (int t : tiles) {
+        if (!t) continue;
+        const int step = piece_tiles(t, pieces), n = (t + step - 1) / step;
+        check(n >= 1 && n <= pieces && (long)step * pieces >= t, "a sequence's own slices cover it", t, pieces, step);
     }
 }
 
@@ -49,7 +61,9 @@ int main() {
         std::vector<int> tiles(B);
         for (int &t : tiles) t = in(0, most);
         const int splits = in(0, 2) ? 64 : in(1, 256);
+        if (splits > 1) walk(tiles, in(1, std::min(4096, B * splits)), in(1, 1024), 0, splits);
         walk(tiles, in(1, std::min(4096, B * splits)), in(1, 1024), in(1, 4), splits);
+        walk_own(tiles, in(1, 4));
     }
     // slices of a plan: waves of a 256-CU GPU, the cap or a row per (sequence, 256 tokens)
     const size_t cap = kWsBytes;
@@ -64,10 +78,18 @@ int main() {
                             const DecodeF32Plan p = plan_f32(nq, per, d, 16, batch, blocks, splits, 4096, 3072);
                             const int64_t parts = std::min<int64_t>(splits, (blocks + 15) / 16);
                             check(p.ws_bytes <= std::max<size_t>(cap, (size_t)row * p.batch * parts), "workspace", (long long)p.ws_bytes, row, batch);
-                            check(p.slots == part_rows(p.slices, p.batch) && p.slices_qf32 <= p.slices && p.slices_qf32 >= 1, "slots");
+                            check(p.slices_qf32 <= p.slices && p.slices_qf32 >= 1, "slices");
+                            const int64_t fit = std::max<int64_t>(1, ((int64_t)cap - 20000) / row);
+                            if (splits == 1) {                   // every sequence its own slices, as many as its partition's waves
+                                check(p.slices == p.batch * p.seq_pieces && p.slots >= (p.seq_pieces > 1 ? p.slices : 1), "own slots");
+                                check(p.seq_pieces <= kSharing && p.seq_pieces >= std::min<int64_t>(std::min<int64_t>(kSharing, (blocks + 1) / 2), fit / p.batch),
+                                      "own slices", p.seq_pieces, blocks, fit);
+                                continue;
+                            }
+                            check(!p.seq_pieces && p.slots == part_rows(p.slices, p.batch), "slots");
                             // half the partial rows of the cap at least, unless the waves or the splits are fewer
-                            const int64_t want = std::min(std::min<int64_t>((4096 + per - 1) / per, p.batch * splits),
-                                                          std::max<int64_t>(1, ((int64_t)cap - 20000) / row / 2));
+                            const int64_t want = std::min(std::min<int64_t>((4096 + per - 1) / per, p.batch * std::min(splits * kSharing, blocks)),
+                                                          std::max<int64_t>(1, fit / 2));
                             check(p.slices >= want, "slices of a wide batch", p.slices, want, batch);
                         }
     std::printf("%ld cases, %ld wrong\n", cases, wrong);

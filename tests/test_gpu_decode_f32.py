@@ -85,6 +85,22 @@ def test_decode_f32_wide_batches(dtype, d, n_kv, group, batch, bad):
     assert pa.error_count() > 0 and pb.error_count() > 0
 
 
+@pytest.mark.parametrize("dtype,d", [(airkv.BF16, 64), (airkv.INT8, 96), (airkv.F32, 224)])
+def test_decode_f32_one_partition(dtype, d):
+    """max_splits 1: a sequence's result does not depend on the others of its
+    batch, bit for bit."""
+    torch = torch_mod()
+    lens = [0, 1, 16, 17, 33, 64, 65, 1000, 300, 2049]
+    cfg = workloads.Config("one", 8, 2, d, 16, dtype, len(lens))
+    _, _, (pool, host, tables, seq_lens, q, _) = _decode_case(cfg, lens, seed=5 + d)
+    q, tables, seq_lens = (torch.from_numpy(x).cuda() for x in (q, tables, seq_lens))
+    out, one = torch.full(q.shape, float("nan"), device="cuda"), torch.full(q.shape, float("nan"), device="cuda")
+    pool.paged_decode(q, tables, seq_lens, out, max_splits=1)
+    for i in range(len(lens)):
+        pool.paged_decode(q[i:i + 1], tables[i:i + 1], seq_lens[i:i + 1], one[i:i + 1], max_splits=1)
+    assert torch.equal(out, one) and bool(torch.isfinite(out).all())
+
+
 @pytest.mark.parametrize("d", [64, 96])
 def test_decode_f32_every_fp8_code(d):
     """Pages written as raw blocks may hold any code: subnormal ones, which the
