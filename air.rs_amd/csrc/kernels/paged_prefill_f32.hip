@@ -54,6 +54,7 @@
 #include "codecs.hpp"
 #include "prefill_common.hpp"
 #include "prefill_rank.hpp"
+#include "prefill_tiles.hpp"
 
 namespace airkv {
 namespace {
@@ -195,15 +196,15 @@ __device__ void slow_column(const PrefillArgs &a, const int32_t *tbl, int kh, in
     auto q_elem = [&](int e) {
         return a.q_dtype == AIR_KV_F32 ? ((const float *)a.q)[qo + e] : bf16_to_f32(((const uint16_t *)a.q)[qo + e]);
     };
-    auto page_row = [&](int t) -> int64_t {
+    auto page_row = [&](uint32_t t) -> int64_t {
         const int32_t blk = tbl[t >> bs_log2];
         if (blk < 0 || blk >= a.num_blocks) return -1;
-        return ((int64_t)blk * a.n_kv_heads + kh) * bs + (t & (bs - 1));
+        return ((int64_t)blk * a.n_kv_heads + kh) * bs + (int)(t & (uint32_t)(bs - 1));
     };
     float m = -INFINITY, l = 0.0f, acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int t0 = 0; t0 < n_keys; t0 += 64) {
+    for (uint32_t t0 = 0; t0 < (uint32_t)n_keys; t0 += 64) {      // (up to 2^31 - 1 keys)
         float s = -INFINITY;
-        if (t0 + lane < n_keys) {
+        if (t0 + lane < (uint32_t)n_keys) {
             const int64_t row = page_row(t0 + lane);
             s = 0.0f;
             for (int e = 0; e < d; ++e)
@@ -220,7 +221,7 @@ __device__ void slow_column(const PrefillArgs &a, const int32_t *tbl, int kh, in
         l = l * alpha + ps;
         m = m_new;
         for (int i = 0; i < 4; ++i) acc[i] *= alpha;
-        const int n = n_keys - t0 < 64 ? n_keys - t0 : 64;
+        const int n = (uint32_t)n_keys - t0 < 64 ? (int)((uint32_t)n_keys - t0) : 64;
         for (int j = 0; j < n; ++j) {
             const float pj = __shfl(p, j);
             const int64_t row = page_row(t0 + j);
@@ -294,7 +295,7 @@ void prefill_f32_kernel(PrefillArgs a) {
     Raw<PT> rk[PASSES], rv[PASSES];
     int32_t id[PASSES];
     uint32_t live = 0;
-    int tile_rows = 0;                                          // NK > 1: rows past these are no wave's, left alone
+    int rows = 0;                                               // NK > 1: rows past these are no wave's, left alone
     auto chunk_row = [&](int i) { return (tid + kThreads * i) / (D / 8); };
     auto chunk_col = [&](int i) { return (tid + kThreads * i) % (D / 8) * 8; };
     // A chunk keeps its place within its block (KT is a multiple of the block
@@ -314,19 +315,18 @@ void prefill_f32_kernel(PrefillArgs a) {
     auto fetch_ids = [&](int t, int kend) {
 #pragma unroll
         for (int i = 0; i < PASSES; ++i) {
-            const int key = t * KT + chunk_row(i);
-            const uint32_t j = (uint32_t)(key < kend ? key : kend - 1) >> bs_log2;
+            const uint32_t j = entry_key(t, KT, chunk_row(i), kend) >> bs_log2;
             id[i] = *reinterpret_cast<const int32_t *>((const char *)tbl + 4 * j);
         }
     };
     auto load_tile = [&](int t, int kend) {
         live = 0;
-        tile_rows = (kend - t * KT + 31) & ~31;
+        rows = tile_rows(t, KT, kend);
 #pragma unroll
         for (int i = 0; i < PASSES; ++i) {
-            if (NK > 1 && chunk_row(i) >= tile_rows) continue;
+            if (NK > 1 && chunk_row(i) >= rows) continue;
             const bool in_pool = id[i] >= 0 && id[i] < a.num_blocks;
-            if (t * KT + chunk_row(i) < kend && in_pool && chunk_col(i) < d) live |= 1u << i;
+            if (tile_key(t, KT, chunk_row(i)) < (uint32_t)kend && in_pool && chunk_col(i) < d) live |= 1u << i;
             const uint32_t blk = in_pool ? id[i] : 0;
             const uint64_t at = (uint64_t)blk * blk_bytes + off[i], sat = (uint64_t)blk * blk_sc + soff[i];
             load_raw<PT>(a.k_pages, a.k_scales, at, sat, rk[i]);
@@ -338,7 +338,7 @@ void prefill_f32_kernel(PrefillArgs a) {
 #pragma unroll
         for (int i = 0; i < PASSES; ++i) {
             if (S::CHUNKS % kThreads != 0 && tid + kThreads * i >= S::CHUNKS) break;
-            if (NK > 1 && chunk_row(i) >= tile_rows) continue;
+            if (NK > 1 && chunk_row(i) >= rows) continue;
             const bool lv = (live >> i) & 1;
             uint8_t *kd = ks + chunk_row(i) * KP + chunk_col(i) * 2;
             uint8_t *vd = vs + chunk_row(i) * VP + chunk_col(i) * 2;
@@ -372,17 +372,17 @@ void prefill_f32_kernel(PrefillArgs a) {
         const int c0 = (n_wg - 1 - w) * S::COLS;                // the workgroup's first column
         const int c_end = c0 + S::COLS < nc ? c0 + S::COLS : nc;
         const int kend = q_offset + (c_end - 1) / G + 1;        // keys the workgroup needs
-        const int nt = (kend + KT - 1) / KT;
+        const int nt = key_tiles(kend, KT);
         const int wc = c0 + 32 * cg;                        // the wave's first column
         const bool wlive = wc < c_end;
         const int col = wc + r32 < c_end ? wc + r32 : c_end - 1;
         const int qr = col / G, h = kh * G + col - qr * G;
         const int qpos = q_offset + qr;
-        // the wave's positions: tiles past the last are skipped, tiles below
-        // the first need no mask (uniform)
-        const int pos_hi = __builtin_amdgcn_readfirstlane(
-            wlive ? q_offset + (wc + 31 < c_end ? wc + 31 : c_end - 1) / G : -1);
-        const int pos_lo = __builtin_amdgcn_readfirstlane(q_offset + (wlive ? wc : c_end - 1) / G);
+        // the wave's positions: tiles at or past the end are skipped, tiles
+        // below the first need no mask (uniform)
+        const uint32_t pos_end = __builtin_amdgcn_readfirstlane(
+            wlive ? q_offset + (wc + 31 < c_end ? wc + 31 : c_end - 1) / G + 1 : 0);
+        const uint32_t pos_lo = __builtin_amdgcn_readfirstlane(q_offset + (wlive ? wc : c_end - 1) / G);
 
         fetch_ids(0, kend);
         // ---- queries, in the B operand's layout (column r32)
@@ -499,15 +499,16 @@ void prefill_f32_kernel(PrefillArgs a) {
         };
         auto compute_tile = [&](int t) {
             const uint8_t *ks = smem + (S::BUFS == 2 ? (t & 1) * S::STAGE : 0), *vs = ks + NP * S::KPART;
-            const int kb = 32 * SUB * kg, k0 = t * KT + kb;      // the wave's first key: of the tile, of the sequence
-            if (k0 > pos_hi) return;                             // behind every row of the wave (uniform)
+            const int kb = 32 * SUB * kg;                        // the wave's first key: of the tile, of the sequence
+            const uint32_t k0 = tile_key(t, KT, kb);
+            if (k0 >= pos_end) return;                           // behind every row of the wave (uniform)
             f32x16 s[SUB];
 #pragma unroll
             for (int u = 0; u < SUB; ++u) s[u] = scores(ks, kb + 32 * u);
             if (k0 + 32 * SUB - 1 > pos_lo) {
 #pragma unroll
                 for (int u = 0; u < SUB; ++u) {
-                    const int kq = qpos - k0 - 32 * u - 4 * hh;
+                    const int kq = (int)((uint32_t)qpos - k0) - 32 * u - 4 * hh;
 #pragma unroll
                     for (int i = 0; i < 16; ++i) s[u][i] = 8 * (i >> 2) + (i & 3) <= kq ? s[u][i] : -INFINITY;
                 }
@@ -723,7 +724,7 @@ hipError_t launch_d(const PrefillArgs &a, int dtype, int32_t max_q_len, hipStrea
 // Sequence lengths are not known here, so the table's width stands for them.
 bool prefill_f32_better(const PrefillArgs &a, int dtype, int32_t max_q_len) {
     const int64_t rows = max_q_len > 0 ? max_q_len : 1;
-    if ((int64_t)a.total_q * a.group > INT32_MAX) return false;      // columns are counted in 32 bits
+    if ((int64_t)a.total_q * a.group > INT32_MAX - 1024) return false;   // columns are counted in 32 bits
     const int64_t wgs = rows * a.batch * a.n_kv_heads * ((a.group + 7) / 8);
     if (wgs > 2560) return true;
     const int d = a.head_dim;
