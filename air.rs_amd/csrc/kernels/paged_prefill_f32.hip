@@ -712,37 +712,6 @@ hipError_t launch_d(const PrefillArgs &a, int dtype, int32_t max_q_len, hipStrea
 
 }  // namespace
 
-// Whether the kernel above beats the vector kernel's prefill (launch_prefill_rows:
-// a workgroup per query row, kv head and eight heads of the group, 64 keys a
-// step), from times fitted to 3360 shapes measured both ways (head_dim 64 to
-// 256, f32 / bf16 / int8 pages, 1 to 128 rows, groups 1 to 8, prefixes 0 to 4096,
-// 1 to 64 (sequence, kv head) pairs; 19 of them are more than 5% slower than
-// the better side).  The vector kernel starts faster (one row without a
-// prefix, head_dim 64: 4.1 us against 6.5; head_dim 256: 6 against 14) and
-// f32 or 1-byte tiles are dear to split, but its work grows with the rows:
-// eight 512-token chunks over bf16 pages of 64 take 2300 us there against 127.
-// Sequence lengths are not known here, so the table's width stands for them.
-bool prefill_f32_better(const PrefillArgs &a, int dtype, int32_t max_q_len) {
-    const int64_t rows = max_q_len > 0 ? max_q_len : 1;
-    if ((int64_t)a.total_q * a.group > INT32_MAX - 1024) return false;   // columns are counted in 32 bits
-    const int64_t wgs = rows * a.batch * a.n_kv_heads * ((a.group + 7) / 8);
-    if (wgs > 2560) return true;
-    const int d = a.head_dim;
-    const double g = a.group <= 2 ? a.group : a.group <= 4 ? 4 : 8;
-    const double steps = (double)(((int64_t)a.max_blocks * a.block_size + 63) / 64 - 1);
-    const double row_step = d <= 64 ? 1.3 + 0.26 * g : d <= 128 ? 2.3 + 0.42 * g : 4.6 + 0.8 * g;
-    const double crowd = wgs > 640 ? 1.0 + (double)(wgs - 640) / 1300 : 1.0;
-    const double t_rows = (3.5 + g + d / 128.0 + row_step * steps) * crowd;
-    const bool split = dtype != AIR_KV_BF16, qf32 = a.q_dtype == AIR_KV_F32;
-    double start, step;                                          // us per launch, per 64 keys
-    if (d <= 64) { start = split ? 7.6 : 6.4; step = split ? 1.75 : 0.87; }
-    else if (d <= 96) { start = split ? 9.8 : 8.6; step = split ? 2.4 : 1.15; }
-    else if (d == 128) { start = 9.8; step = 4.2; }
-    else { start = split ? 15.5 : qf32 ? 19.0 : 14.0; step = split ? 10.0 : qf32 ? 7.6 : 3.7; }
-    if (qf32) start += 1.0;
-    return start + step * steps < t_rows;
-}
-
 hipError_t launch_prefill_f32(PrefillArgs a, int dtype, int32_t max_q_len, int cus, hipStream_t s) {
     a.max_len = (int64_t)a.max_blocks * a.block_size;
     a.ns_max = 1;

@@ -5,8 +5,8 @@
 // A workgroup owns one (query row, kv head, sequence) and the query heads that
 // share the kv head (GQA, src/chunked_attn.rs:240-243), G of them at a time:
 // groups of up to 8 heads take one workgroup per kv head (G the next power of
-// two, heads past the group masked), larger groups ceil(group / 8) workgroups
-// of 8 heads each.  It runs an online softmax over the row's causal keys in
+// two, heads past the group masked), larger groups ceil(group / G) workgroups
+// of G heads each.  It runs an online softmax over the row's causal keys in
 // 64-token tiles and writes the normalised output.
 //
 // Thread mapping: head_dim/8 lanes cover one token row, 8 elements per lane,
@@ -344,13 +344,14 @@ hipError_t launch_d(const PrefillArgs &a, hipStream_t s) {
     return launch_typed<DT, G, 256>(a, s);
 }
 
-// Heads per workgroup: the group rounded up to a power of two, at most 8.
+// Heads per workgroup: the group rounded up to a power of two, at most 8 (4 up to
+// head_dim 128, where larger groups only come here past 2^31 columns).
 template <int DT>
 hipError_t launch_g(const PrefillArgs &a, hipStream_t s) {
     if (a.group == 1) return launch_d<DT, 1>(a, s);
     if (a.group == 2) return launch_d<DT, 2>(a, s);
-    if (a.group <= 4) return launch_d<DT, 4>(a, s);
-    return launch_d<DT, 8>(a, s);
+    if (a.group <= 4 || a.head_dim <= 128) return launch_d<DT, 4>(a, s);
+    return launch_typed<DT, 8, 256>(a, s);
 }
 
 }  // namespace

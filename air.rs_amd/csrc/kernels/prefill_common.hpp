@@ -56,7 +56,5 @@ hipError_t launch_prefill(PrefillArgs a, int dtype, int block_size, int32_t max_
 hipError_t launch_prefill_f32(PrefillArgs a, int dtype, int32_t max_q_len, int cus, hipStream_t s);
 // One query row at a time on the vector units, for the same pools.
 hipError_t launch_prefill_rows(PrefillArgs a, int dtype, int32_t max_q_len, hipStream_t s);
-// Which of the two this launch is faster on.
-bool prefill_f32_better(const PrefillArgs &a, int dtype, int32_t max_q_len);
 
 }  // namespace airkv

@@ -8,6 +8,7 @@
 
 #include "host/status.hpp"
 #include "kernels/prefill_common.hpp"
+#include "kernels/prefill_rule.hpp"
 #include "pool.hpp"
 
 using airkv::fail;
@@ -258,7 +259,9 @@ int air_paged_prefill(air_kv_pool *p, void *stream, const void *q, int32_t q_dty
         // F32 pages, head_dim other than 128: the f32-precision kernel, or
         // for launches too small for it the vector kernel
         if (batch > 65535) return fail(AIR_KV_E_INVALID_ARG, "batch %d above 65535 for this pool", batch);
-        hipError_t e = airkv::prefill_f32_better(a, d.dtype, max_q_len)
+        const airkv::PrefillShape shape = {d.dtype, d.head_dim, d.n_kv_heads, a.group, q_dtype, total_q, batch,
+                                           max_q_len, (int64_t)max_blocks * d.block_size};
+        hipError_t e = airkv::prefill_f32_better(shape)
                            ? airkv::launch_prefill_f32(a, d.dtype, max_q_len, p->cus, (hipStream_t)stream)
                            : airkv::launch_prefill_rows(a, d.dtype, max_q_len, (hipStream_t)stream);
         return e == hipSuccess ? AIR_KV_OK : hip_fail(e, "air_paged_prefill launch");
@@ -275,6 +278,13 @@ int air_paged_prefill(air_kv_pool *p, void *stream, const void *q, int32_t q_dty
     }
     hipError_t e = airkv::launch_prefill(a, d.dtype, d.block_size, max_q_len, p->cus, (hipStream_t)stream);
     return e == hipSuccess ? AIR_KV_OK : hip_fail(e, "air_paged_prefill launch");
+}
+
+// The rule of the pools above, for the tests: 1 where the f32-precision kernel
+// runs, 0 where the row kernel does.
+int airkv_prefill_f32_better(int32_t dtype, int32_t head_dim, int32_t n_kv_heads, int32_t group, int32_t q_dtype,
+                             int32_t total_q, int32_t batch, int32_t max_q_len, int64_t tokens) {
+    return airkv::prefill_f32_better({dtype, head_dim, n_kv_heads, group, q_dtype, total_q, batch, max_q_len, tokens});
 }
 
 int air_kv_copy_blocks(air_kv_pool *p, void *stream, const int32_t *src, const int32_t *dst, int32_t n) {

@@ -78,10 +78,11 @@ def test_prefill_matches_oracle_small(dtype, group):
     (airkv.BF16, 64, 2, 4, 16), (airkv.BF16, 96, 2, 2, 32), (airkv.BF16, 256, 1, 8, 16),
     (airkv.INT8, 160, 2, 2, 16), (airkv.FP8, 32, 4, 1, 32), (airkv.INT8, 224, 1, 12, 16)])
 def test_prefill_vector_path_vs_oracle(dtype, head_dim, n_kv, group, bs):
-    """Pools the matrix-core prefill does not take -- f32 pages (the
-    reference's own cache dtype) and head_dim other than 128 -- run each
-    query row on the split kernel over its causal keys: the oracle's
-    blockwise attention, within the same tolerance."""
+    """Pools the 128 matrix-core prefill does not take -- f32 pages (the
+    reference's own cache dtype) and head_dim other than 128 -- run at f32
+    precision, on the matrix cores or row by row: the oracle's blockwise
+    attention, within the same tolerance.  (test_gpu_prefill_f32.py holds
+    the edges of both kernels.)"""
     cfg = workloads.Config("vec", n_kv * group, n_kv, head_dim, bs, dtype, 4)
     got, want = _prefill_case(cfg, [1, 37, 300, 700], [1, 37, 64, 100], seed=97 + head_dim)
     err = rel_err(got, want)

@@ -2,7 +2,10 @@
 oracle's blockwise attention, at the edges of its tiles: columns (query rows
 times the GQA group) around a wave's 32 and a workgroup's 32 to 128, keys around
 the 32- to 128-key tiles, head_dim below each built size, and launches whose
-waves share a column set's keys four, two and one ways."""
+waves share a column set's keys four, two and one ways; and the row-by-row kernel
+that small launches of these pools take, on each of its builds."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -48,6 +51,31 @@ def test_prefill_f32_tile_edges(dtype, d, n_kv, group, bs, q_lens, ctx, q_bf16):
     err = rel_err(got, want)
     log(f"prefill f32 dtype={dtype} d={d} group={group} q_bf16={q_bf16}: rel err {err:.2e}")
     assert err <= TOL_F32
+
+
+def _rule(dtype, d, n_kv, group, q_bf16, q_lens, tokens):
+    """Whether such a launch takes the f32-precision kernel (else the row kernel)."""
+    f = airkv.load().airkv_prefill_f32_better
+    f.argtypes = [ctypes.c_int32] * 8 + [ctypes.c_int64]
+    return f(dtype, d, n_kv, group, airkv.BF16 if q_bf16 else airkv.F32, sum(q_lens), len(q_lens), max(q_lens), tokens)
+
+
+# (head_dim, kv heads, group): every width and head count the row kernel is built for
+ROWS = [(32, 4, 1), (64, 2, 2), (64, 1, 4), (32, 1, 3), (96, 4, 1), (96, 2, 2), (96, 1, 4), (160, 4, 1), (256, 2, 2),
+        (224, 1, 3), (192, 1, 8), (256, 1, 12)]
+
+
+@pytest.mark.parametrize("dtype,d,n_kv,group,q_bf16",
+                         [(dt, d, kv, g, qb) for dt in (airkv.F32, airkv.BF16, airkv.INT8, airkv.FP8) for d, kv, g in ROWS
+                          for qb in (False, True) if not qb or (g == 1 and d != 32)] +
+                         [(airkv.F32, 128, kv, g, False) for kv, g in ((4, 1), (2, 2), (1, 4))])
+def test_prefill_rows_small_chunks(dtype, d, n_kv, group, q_bf16):
+    """Chunks of 1 to 8 rows over 0 to 61 tokens before them: the row kernel."""
+    q_lens, ctx = [8, 5, 1, 3], [40, 5, 64, 20]
+    assert not _rule(dtype, d, n_kv, group, q_bf16, q_lens, 64)
+    cfg = workloads.Config("rows", n_kv * group, n_kv, d, 16, dtype, len(ctx))
+    got, want = _prefill_case(cfg, ctx, q_lens, seed=43 + d + group, q_bf16=q_bf16)
+    assert rel_err(got, want) <= TOL_F32
 
 
 @pytest.mark.parametrize("dtype,d", [(airkv.BF16, 64), (airkv.F32, 64), (airkv.F32, 128)])
