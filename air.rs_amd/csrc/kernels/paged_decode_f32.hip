@@ -506,9 +506,9 @@ void decode_f32_kernel(DecodeArgs a) {
         }
         float mt = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
         mt = max_x32(max_x16(mt));
-        // the running max follows only when a tile exceeds it by 2^8 (see
-        // paged_decode_mfma.hip)
-        if (__ballot(mt > m_run + 8.0f) != 0ull) {
+        // (no slack here: probabilities above 1 would overflow on values near
+        // the largest f32)
+        if (__ballot(mt > m_run) != 0ull) {
             const float m_new = fmaxf(m_run, mt);
             const float alpha = (m_run == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
             l_run *= alpha;

@@ -136,3 +136,43 @@ def test_decode_f32_every_fp8_code(d):
     want = host.paged_decode(q, tables, np.array([n // bs * bs], np.int32), chunk=64)
     assert rel_err(out.cpu().numpy(), want) <= TOL_F32
     assert pool.error_count(reset=True) > 0
+
+
+@pytest.mark.parametrize("d", [64, 256])
+@pytest.mark.parametrize("dtype", [airkv.F32, airkv.BF16])
+@pytest.mark.parametrize("case", ["huge", "tiny", "tiny_k", "tiny_q"])
+def test_decode_f32_value_ranges(dtype, d, case):
+    """Values near the largest f32 (scores grow along the sequence, so a later
+    tile's probabilities are the largest), values and keys near the least normal
+    one (keys against queries as large), against 64 bits."""
+    torch = torch_mod()
+    n, kv, group = 400, 2, 2
+    cfg = workloads.Config("range", kv * group, kv, d, 16, dtype, 1)
+    w, pool, _, host, tables, lens, _, _ = _setup(cfg, [n - 1], seed=3)
+    rng = np.random.default_rng(4)
+    k, v = (rng.standard_normal((n, kv, d)).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((1, kv * group, d)).astype(np.float32)
+    if case == "huge":
+        v = (v * np.float32(1e35) + np.float32(1e36)).astype(np.float32)
+        k[:, :, 0] = np.arange(n)[:, None] / 16 * np.sqrt(d)        # one nat per tile
+        q[:, :, 0] = 1.0
+    elif case == "tiny":
+        v *= np.float32(1e-36)
+    elif case == "tiny_k":
+        k, q = k * np.float32(1e-35), q * np.float32(1e35)
+    else:
+        k, q = k * np.float32(1e35), q * np.float32(1e-35)
+    slots = (tables[0, np.arange(n) // 16].astype(np.int64) * 16 + np.arange(n) % 16)
+    pool.append(torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda(), torch.from_numpy(slots).cuda())
+    qt, lens = torch.from_numpy(q).cuda(), np.array([n], np.int32)
+    if dtype == airkv.BF16:
+        k, v = (torch.from_numpy(x).to(torch.bfloat16).float().numpy() for x in (k, v))
+    s = np.einsum("gd,ngd->gn", q[0].astype(np.float64), np.repeat(k, group, 1).astype(np.float64)) / np.sqrt(d)
+    p = np.exp(s - s.max(1, keepdims=True))
+    want = np.einsum("gn,ngd->gd", p / p.sum(1, keepdims=True), np.repeat(v, group, 1).astype(np.float64))
+    for most in (64, 1):
+        out = torch.full(q.shape, float("nan"), device="cuda")
+        pool.paged_decode(qt, torch.from_numpy(tables).cuda(), torch.from_numpy(lens).cuda(), out, max_splits=most)
+        err = float(np.abs(out.cpu().numpy()[0].astype(np.float64) - want).max() / np.abs(want).max())
+        log(f"decode f32 {case} dtype={dtype} d={d}: rel err {err:.2e}")
+        assert err <= TOL_F32
