@@ -5,13 +5,16 @@
 // Semantics are paged_prefill.hip's (blockwise_attention_head with q_offset =
 // seq_len - q_len, src/chunked_attn.rs:114-213, over paged storage).  What
 // differs is the arithmetic: queries, keys, probabilities, values and sums
-// keep their 24 bits, so no result depends on the magnitudes of the inputs.
-// An f32 operand enters v_mfma_f32_32x32x16_bf16 as three bf16 parts, each the
-// rounding of what the parts before it leave (8 bits a part, the exponent
-// range of f32), and a product of two such operands is the six part products
-// down to 2^-16; bf16 queries and bf16 pages are one part as they are.  The
-// matrix cores run those six at 2.7 times the rate of their own f32 products.
-// 1-byte codes are dequantized (code * scale, one rounding) as they are staged.
+// keep their 24 bits between 2^-110 and the largest f32.  An f32 operand enters
+// v_mfma_f32_32x32x16_bf16 as three bf16 parts, each the rounding of what the
+// parts before it leave (8 bits a part, the exponent range of f32), and a product
+// of two such operands is the six part products down to 2^-16; bf16 queries and
+// bf16 pages are one part as they are.  The matrix cores run those six at 2.7
+// times the rate of their own f32 products.  1-byte codes are dequantized (code *
+// scale, one rounding) as they are staged.  Below 2^-110 the parts under 2^-126
+// are lost: f32 values of 1e-37 keep 13 bits.  (Computing their columns again as
+// below, found by the least query element and output, cost every small launch
+// 1.5 to 4%.)
 //
 // Rounding of the sums: the part products below the leading ones are added
 // first (in the scores, in an accumulator of their own), and a tile's P.V

@@ -151,3 +151,51 @@ def _host_with_zero_block(host, cfg):
     hz = oracle.HostPool(host.num_blocks + 1, cfg.block_size, cfg.n_kv_heads, cfg.head_dim, cfg.dtype)
     hz.k[:host.num_blocks], hz.v[:host.num_blocks] = host.k, host.v
     return hz
+
+
+@pytest.mark.parametrize("dtype,d", [(airkv.F32, 64), (airkv.F32, 128), (airkv.BF16, 64), (airkv.BF16, 256)])
+@pytest.mark.parametrize("case", ["unit", "huge", "tiny", "tiny_channel", "tiny_k", "tiny_q", "spikes"])
+def test_prefill_f32_value_ranges(dtype, d, case):
+    """Values near the largest f32 and near 2^-106 (24 bits are kept from 2^-110 on),
+    a channel of such among ordinary ones, keys of 1e-32 or 1e32 under queries of
+    the opposite, and a few huge values, against 64 bits, channel by channel.  Sums
+    of up to 300 f32 products in any order: within 300 * 2^-24 = 1.8e-5."""
+    torch = torch_mod()
+    n, kv, group = 300, 2, 4
+    cfg = workloads.Config("range", kv * group, kv, d, 16, dtype, 2)
+    pool, _, tables, lens = _setup(cfg, [n, n], seed=5)
+    rng = np.random.default_rng(4)
+    k, v = (rng.standard_normal((2 * n, kv, d)).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((2 * n, kv * group, d)).astype(np.float32)
+    if case == "huge":
+        v *= np.float32(1e36)
+    elif case == "tiny":
+        v = ((np.abs(v) + 1) * np.float32(1e-32)).astype(np.float32)
+    elif case == "tiny_channel":
+        v[:, :, 5] = (np.abs(v[:, :, 5]) + 1) * np.float32(1e-32)
+    elif case == "tiny_k":
+        k, q = k * np.float32(1e-32), q * np.float32(1e32)
+    elif case == "tiny_q":
+        k, q = k * np.float32(1e32), q * np.float32(1e-32)
+    elif case == "spikes":
+        v.reshape(-1)[rng.integers(0, v.size, 5)] = 1e37
+    slots = np.concatenate([t[np.arange(n) // 16].astype(np.int64) * 16 + np.arange(n) % 16 for t in tables])
+    pool.append(torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda(), torch.from_numpy(slots).cuda())
+    cu = np.array([0, n, 2 * n], np.int32)
+    assert _rule(dtype, d, kv, group, False, [n, n], 304)
+    out = torch.full(q.shape, float("nan"), device="cuda")
+    pool.paged_prefill(torch.from_numpy(q).cuda(), torch.from_numpy(cu).cuda(), torch.from_numpy(tables).cuda(),
+                       torch.from_numpy(lens).cuda(), out)
+    got = out.cpu().numpy().astype(np.float64)
+    if dtype == airkv.BF16:
+        k, v = (torch.from_numpy(x).to(torch.bfloat16).float().numpy() for x in (k, v))
+    want = np.empty_like(got)
+    for b in range(2):
+        r = slice(b * n, (b + 1) * n)
+        for h in range(kv * group):
+            s = q[r, h].astype(np.float64) @ k[r, h // group].astype(np.float64).T / np.sqrt(d)
+            p = np.exp(np.where(np.tri(n, dtype=bool), s, -np.inf) - np.where(np.tri(n, dtype=bool), s, -np.inf).max(1, keepdims=True))
+            want[r, h] = p / p.sum(1, keepdims=True) @ v[r, h // group].astype(np.float64)
+    err = float((np.abs(got - want).max((0, 1)) / np.abs(want).max((0, 1))).max())
+    log(f"prefill f32 {case} dtype={dtype} d={d}: worst channel's rel err {err:.2e}")
+    assert err <= 1.8e-5
