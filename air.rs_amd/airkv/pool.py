@@ -210,8 +210,8 @@ class KvPool:
                             max_splits=64, workspace=None, stream=None):
         """One decode step: append k_new / v_new (float32 [batch, n_kv_heads,
         head_dim]) as each sequence's token seq_lens[b] - 1, then attend as
-        paged_decode, in one launch (INT8 / FP8 rows quantized as append
-        quantizes them)."""
+        paged_decode, in one call (INT8 / FP8 rows quantized as append
+        quantizes them).  No other sequence of the call may read that token."""
         head, tail = self._decode_args(q, block_tables, seq_lens, out, scale, max_splits, workspace, stream)
         rows = self._new_rows(q, k_new, v_new)
         _lib.check(_lib.load().air_paged_decode_append(*head, *rows, *tail), "air_paged_decode_append")

@@ -38,9 +38,9 @@
 // Bound by the page loads where the matrix cores keep up (f32 pages, bf16
 // pages under bf16 queries), by the f32 products and the widening on 1-byte
 // pages.  48 sequences of 256 to 4096 tokens, 32 heads over 8: bf16 pages of 64
-// 48.8 us, 4.73 TB/s, 41 of them the slices' (180 us on the vector kernel this
-// replaced, four launches); f32 pages of 64 87 us, 5.3 TB/s (194); 64 sequences
-// of 256 to 8192 over int8 pages of 64 155 us, 2.2 TB/s (453).
+// 49 us, 4.7 TB/s, 41 of them the slices' (180 us on the vector kernel this
+// replaced, four launches); f32 pages of 64 88 us, 5.2 TB/s (204); 64 sequences
+// of 256 to 8192 over int8 pages of 64 151 us, 2.3 TB/s (449).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

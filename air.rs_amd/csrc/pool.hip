@@ -257,7 +257,7 @@ int air_paged_prefill(air_kv_pool *p, void *stream, const void *q, int32_t q_dty
     a.ws_units = 0;
     if (!airkv::prefill_supported(d.dtype, d.head_dim, d.block_size, d.scale_group)) {
         // F32 pages, head_dim other than 128: the f32-precision kernel, or
-        // for launches too small for it the vector kernel
+        // for launches too small for it the row kernel
         if (batch > 65535) return fail(AIR_KV_E_INVALID_ARG, "batch %d above 65535 for this pool", batch);
         const airkv::PrefillShape shape = {d.dtype, d.head_dim, d.n_kv_heads, a.group, q_dtype, total_q, batch,
                                            max_q_len, (int64_t)max_blocks * d.block_size};

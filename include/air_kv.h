@@ -275,14 +275,17 @@ int air_paged_decode(air_kv_pool *pool, void *stream, const void *q, int32_t q_d
                      int32_t batch, int32_t max_blocks, float scale, int32_t max_splits,
                      void *workspace, size_t ws_bytes, void *out, int32_t out_dtype);
 
-/* One decode step's append and attention in one launch: the same pages and
+/* One decode step's append and attention in one call: the same pages and
  * outputs as air_kv_append of k_new / v_new (f32, [batch][n_kv_heads]
  * [head_dim]) at each sequence's token seq_lens[b] - 1 -- the slot its block
  * table gives that token, the slot SequenceManager::append_token hands out
  * (src/paged_attention.rs:225-248) -- followed by air_paged_decode with the
  * same arguments (the reference's decode step appends the token's K/V, then
  * attends, src/model.rs:577, src/ops.rs:333-357).  Each new row is written by
- * the wave that attends over it, so no launch orders the two.  Sequences of
+ * the wave that attends over it, so no launch orders the two: no other sequence
+ * of the call may read the token a sequence appends (a block that is written is
+ * held by one sequence, as copy-on-write before the step leaves it; several rows
+ * of one table take air_kv_append, then air_paged_decode).  Sequences of
  * length 0 append nothing; a sequence longer than its table, or whose last
  * block is outside the pool, appends nothing and is counted as by
  * air_paged_decode.  New rows of INT8 / FP8 pools are quantized exactly as

@@ -69,8 +69,8 @@ def test_decode_matches_oracle_small(dtype, group):
 def test_decode_groups_above_16(dtype, n_kv, group):
     """Query heads per kv head beyond the matrix-core kernel's 16 (multi-query
     attention: one kv head for all heads; the reference takes any ratio,
-    src/chunked_attn.rs:65-72): the split kernel serves the group eight heads
-    per workgroup, the last workgroup's heads past the group masked."""
+    src/chunked_attn.rs:65-72): the f32-precision kernel serves the group 16
+    heads to a wave, the last wave's heads past the group masked."""
     log(f"decode group {group} dtype={dtype}")
     cfg = workloads.Config("mqa", n_kv * group, n_kv, 128, 16, dtype, 4)
     got, want, _ = _decode_case(cfg, [5, 64, 333, 900], seed=90 + group)
@@ -83,7 +83,7 @@ def test_decode_groups_above_16(dtype, n_kv, group):
                                                   (airkv.FP8, 224, 3), (airkv.BF16, 192, 16)])
 def test_decode_other_head_dims(dtype, head_dim, group):
     """head_dim a multiple of 32 that is not 64, 128 or 256 (the pool takes any
-    up to 256): the split kernel's lanes past head_dim idle."""
+    up to 256): the columns past head_dim read as zeros."""
     log(f"decode head_dim {head_dim} dtype={dtype} group={group}")
     cfg = workloads.Config("hd", 2 * group, 2, head_dim, 16, dtype, 4)
     got, want, _ = _decode_case(cfg, [3, 70, 257, 640], seed=110 + head_dim)
@@ -189,7 +189,7 @@ def test_pieces_per_sequence_capped_by_max_splits(dtype, max_splits):
 def test_quantized_pool_geometries(dtype, head_dim, scale_group):
     """1-byte pools of every geometry: head_dim 128 with scale groups of 32 or
     more takes the matrix-core kernel, the others (head_dim 64 / 256, groups
-    of 16) the vector kernel; both against the oracle on the dequantized
+    of 16) the f32-precision kernel; both against the oracle on the dequantized
     cache."""
     cfg = workloads.Config("qgeo", 16, 2, head_dim, 16, dtype, 4, scale_group=scale_group)
     got, want, _ = _decode_case(cfg, [5, 300, 1000, 64], seed=47 + head_dim + scale_group)

@@ -9,8 +9,8 @@ that takes two launches, GQA groups 1, 2, 4, 8 and 16, bf16 and f32 queries, pag
 16 and 32, a sequence of length 0, a last block outside the pool, a sequence
 longer than its table, repeated calls, int8 (Q8_0) and fp8 pools (the new
 rows quantized in the launch: codes and scales bit-exact with air_kv_append
-and with the oracle), and pools off the matrix-core decode (f32 pages, other
-head dims, small scale groups, groups above 16: append, then decode)."""
+and with the oracle), and pools off the 128 matrix-core decode (f32 pages, other
+head dims, small scale groups, groups above 16)."""
 import numpy as np
 import pytest
 
@@ -211,7 +211,7 @@ def test_decode_append_batch_above_one_launch():
 def test_decode_append_skips_invalid_sequences(dtype):
     """Length 0, a last block outside the pool and a sequence longer than its
     table append nothing, as the reference path appends nothing for them (the
-    matrix-core step on bf16 pages, the vector path's slots on f32 pages)."""
+    128 kernel on bf16 pages, the f32-precision one on f32 pages)."""
     log(f"decode_append invalid sequences dtype={dtype}")
     ctx = [50, 63, 200, 17, 90]
     cfg = workloads.Config("decode_append_bad", 32, 8, 128, 16, dtype, len(ctx))
@@ -257,13 +257,12 @@ def test_decode_append_repeat_is_stable():
                                                           (airkv.BF16, 32, 64, 16, 32), (airkv.F32, 32, 128, 16, 32),
                                                           (airkv.BF16, 192, 128, 32, 32), (airkv.F32, 16, 96, 32, 32)])
 def test_decode_append_vector_path_pools(dtype, n_q, head_dim, bs, group):
-    """Pools off the matrix-core decode -- f32 pages, head_dim 64 or 96, 1-byte
-    pages with scale groups of 16, 24 query heads per kv head -- take the
-    same entry point: each sequence's slot from its table, the rows appended
-    by air_kv_append's kernel, then the split decode.  Pages, scales and
-    outputs equal air_kv_append + air_paged_decode bit for bit, the pages and
-    scales the oracle's append."""
-    log(f"decode_append vector path dtype={dtype} n_q={n_q} d={head_dim} bs={bs} scale_group={group}")
+    """Pools off the 128 matrix-core decode -- f32 pages, head_dim 64 or 96, 1-byte
+    pages with scale groups of 16, 24 query heads per kv head -- take the same
+    entry point on the f32-precision kernel, which writes the rows itself.
+    Pages, scales and outputs equal air_kv_append + air_paged_decode bit for bit,
+    the pages and scales the oracle's append."""
+    log(f"decode_append f32 precision dtype={dtype} n_q={n_q} d={head_dim} bs={bs} scale_group={group}")
     ctx = [0, 15, 31, 200, 1500]
     cfg = workloads.Config("decode_append_vec", n_q, 8, head_dim, bs, dtype, len(ctx), scale_group=group)
     w, pa, pb, host, tables, lens, k_new, v_new = _setup(cfg, ctx, seed=201 + dtype + head_dim)
@@ -274,3 +273,18 @@ def test_decode_append_vector_path_pools(dtype, n_q, head_dim, bs, group):
     log(f"  identical to append + decode; rel err vs oracle {err:.2e}")
     assert err <= (1e-3 if dtype in (airkv.F32, airkv.BF16) else 2e-2)
     assert pa.error_count() == 0 and pb.error_count() == 0
+
+
+@pytest.mark.parametrize("batch,bad", [(256, 70), (257, 256)])
+def test_decode_append_scan_edges(batch, bad):
+    """Both sides of the 256 sequences that one wave scans alone, with one longer
+    than its table: it appends nothing and is counted."""
+    ctx = [(11 * i) % 50 for i in range(batch)]
+    cfg = workloads.Config("decode_append_scan", 4, 1, 128, 16, airkv.BF16, batch)
+    w, pa, pb, host, tables, lens, k_new, v_new = _setup(cfg, ctx, seed=101 + batch)
+    lens[bad] = tables.shape[1] * 16 + 5
+    mask = np.arange(batch) != bad
+    q = np.random.default_rng(103).standard_normal((batch, 4, 128)).astype(np.float32)
+    q, got = _run_pair(cfg, pa, pb, host, tables, lens, k_new, v_new, q, q_f32=False, append_mask=mask)
+    assert rel_err(got[mask], host.paged_decode(q[mask], tables[mask], lens[mask], chunk=64)) <= TOL_BF16
+    assert pa.error_count() > 0 and pb.error_count() > 0

@@ -6,8 +6,8 @@ checked bit for bit against the same eager calls on a twin pool (outputs,
 pages and group scales), with new query / K / V values written in place
 before each replay and other eager launches and synchronisations between
 the replays.  bf16 pools (one matrix-core launch), int8 pools (the new rows
-quantized in that launch) and f32 pools (the vector path: slots, append,
-decode and merge kernels in the graph).  The paged prefill with its key
+quantized in that launch) and f32 pools (the f32-precision kernel and its
+merge in the graph).  The paged prefill with its key
 split (plan, main and merge kernels) and the gather replay the same way."""
 import numpy as np
 import pytest

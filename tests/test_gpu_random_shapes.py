@@ -12,8 +12,8 @@ included), query and output dtypes.  Each case checks, through the C ABI:
   * the paged prefill of the newest rows of a few sequences (chunks of 0 ..
     32 rows) within tolerance of the oracle's blockwise attention.
 
-Whichever kernels a shape selects (matrix-core or vector decode and
-prefill, fused or appended step) must agree with the oracle."""
+Whichever kernels a shape selects (the 128 or the f32-precision decode and
+prefill, row by row, fused or appended step) must agree with the oracle."""
 import numpy as np
 import pytest
 
