@@ -369,8 +369,11 @@ void decode_f32_kernel(DecodeArgs a) {
             __builtin_amdgcn_s_waitcnt(0);               // written before the loads below are issued
             asm volatile("" ::: "memory");
         }
-        const __amdgpu_buffer_rsrc_t rk = rsrc((const char *)a.k_pages + row0 * d * EB, 16 * d * EB);
-        rv = rsrc((const char *)a.v_pages + row0 * d * EB, 16 * d * EB);
+        // rows past the sequence, and a block outside the pool, read as zeros
+        // without a memory access
+        const int nv = ok ? __builtin_amdgcn_readlane(nv_l, idx) : 0;
+        const __amdgpu_buffer_rsrc_t rk = rsrc((const char *)a.k_pages + row0 * d * EB, nv * d * EB);
+        rv = rsrc((const char *)a.v_pages + row0 * d * EB, nv * d * EB);
         if (lines) {
             // line column c: words 8 c .. + 8 of kw, one 16-byte load each half
 #pragma unroll
@@ -386,8 +389,8 @@ void decode_f32_kernel(DecodeArgs a) {
             }
         }
         if constexpr (kByte<PT>) {
-            const __amdgpu_buffer_rsrc_t rks = rsrc(a.k_scales + row0 * n_sc, 16 * n_sc * 4);
-            rvs = rsrc(a.v_scales + row0 * n_sc, 16 * n_sc * 4);
+            const __amdgpu_buffer_rsrc_t rks = rsrc(a.k_scales + row0 * n_sc, nv * n_sc * 4);
+            rvs = rsrc(a.v_scales + row0 * n_sc, nv * n_sc * 4);
 #pragma unroll
             for (int m = 0; m < KM; ++m)
                 ksc[m] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
@@ -526,13 +529,8 @@ void decode_f32_kernel(DecodeArgs a) {
             constexpr int p = decltype(pc)::value, SZ = P::size(p);
             float x[4][SZ];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < 4; ++i)
                 widen<PT, SZ, FF>(vw[i][p], kByte<PT> ? vsc[kByte<PT> ? i : 0][kByte<PT> ? p : 0] : 1.0f, x[i]);
-                // rows past the sequence hold stale bytes, perhaps not finite
-                if (!full)
-#pragma unroll
-                    for (int j = 0; j < SZ; ++j) x[i][j] = 4 * g4 + i < nv ? x[i][j] : 0.0f;
-            }
 #pragma unroll
             for (int j = 0; j < SZ; ++j) {
                 const f32x4 o0 = mfma4(x[1][j], pr[1], mfma4(x[0][j], pr[0], zero));
