@@ -16,6 +16,9 @@ namespace airkv {
 
 constexpr int kMaxBatch = 4096;            // sequences per launch (the host splits larger batches)
 
+// ceil(n / m) of counts up to 2^31 - 1.
+AIRKV_HD inline int ceil_div(int n, int m) { return (int)(((uint32_t)n + (uint32_t)m - 1) / (uint32_t)m); }
+
 // Tiles per slice: an equal share of `total` over the resident waves, but at
 // least full_chunk once every SIMD has a wave (simd_slices per kv head), and
 // large enough that no sequence meets more than max_splits slices.  A sequence
@@ -23,8 +26,8 @@ constexpr int kMaxBatch = 4096;            // sequences per launch (the host spl
 // chunk >= ceil((T - 1) / (max_splits - 1)) for the longest sequence (tmax tiles)
 // bounds every one; max_splits 1 leaves one slice per kv head.
 AIRKV_HD inline int slice_chunk(int total, int slices, int simd_slices, int full_chunk, int tmax, int max_splits) {
-    const int lone = (total + simd_slices - 1) / simd_slices;
-    int c = (total + slices - 1) / slices;
+    const int lone = ceil_div(total, simd_slices);
+    int c = ceil_div(total, slices);
     const int least = lone < full_chunk ? lone : full_chunk;
     c = c > least ? c : least;
     c = c > 1 ? c : 1;
@@ -46,7 +49,7 @@ AIRKV_HD inline int shared_tiles(int t) {
 
 // Its tiles per slice (max_splits at least 2; simd_slices give every SIMD a wave).
 AIRKV_HD inline int shared_chunk(int total, int slices, int simd_slices, int tmax, int max_splits) {
-    int c = (total + slices - 1) / slices;
+    int c = ceil_div(total, slices);
     c = c > 1 ? c : 1;
     const int part = (tmax - 1 + max_splits - 2) / (max_splits - 1);          // slice_chunk's, by partitions
     if (part <= c) return c;
@@ -54,8 +57,8 @@ AIRKV_HD inline int shared_chunk(int total, int slices, int simd_slices, int tma
     int cs = (tmax - 1 + most - 1) / most;                                    // and by their slices
     cs = cs > shared_tiles(tmax) ? cs : shared_tiles(tmax);
     // a few slices more than SIMDs: the SIMDs with two would end last
-    const int lone = (total + simd_slices - 1) / simd_slices;
-    if (cs < lone && 3 * cs > 2 * lone) cs = lone;
+    const int lone = ceil_div(total, simd_slices);
+    if (cs < lone && cs > lone / 3 * 2) cs = lone;
     cs = cs < part ? cs : part;
     return c > cs ? c : cs;
 }
@@ -105,7 +108,8 @@ inline DecodeF32Plan plan_f32(int64_t n_q_heads, int64_t per_slice, int64_t d, i
     // lengths are 32-bit: a wider table's rest is never reached
     const int64_t tiles_per_seq = max64(1, min64((max_blocks * block_size + 15) / 16, ((int64_t)INT32_MAX + 15) / 16));
     DecodeF32Plan pl;
-    const int64_t nb = pl.batch = max64(1, min64(min64(batch, kMaxBatch), INT32_MAX / tiles_per_seq));
+    // tiles of a launch in 32 bits, with room for the windows of 64 past the last
+    const int64_t nb = pl.batch = max64(1, min64(min64(batch, kMaxBatch), (INT32_MAX - 65536) / tiles_per_seq));
     const int64_t parts = min64(max_splits, (tiles_per_seq + 15) / 16);
     const size_t row = (size_t)n_q_heads * (d + 2) * 4, wide = row * nb * parts;
     const size_t rest = decode_align256((size_t)(nb + 2) * 4) + 256;     // the prefix and the alignment of the sums

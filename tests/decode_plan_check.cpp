@@ -65,6 +65,20 @@ int main() {
         walk(tiles, in(1, std::min(4096, B * splits)), in(1, 1024), in(1, 4), splits);
         walk_own(tiles, in(1, 4));
     }
+    // the widest launches: tile counts up to the plan's bound
+    for (int64_t blocks : {(int64_t)INT32_MAX, (int64_t)(1 << 27), (int64_t)(1 << 26) - 1, (int64_t)(1 << 20) + 7, (int64_t)524288})
+        for (int batch : {1, 3, 15, 16, 31, 4096}) {
+            ++cases;
+            const DecodeF32Plan p = plan_f32(8, 8, 64, 16, batch, blocks, 64, 4096, 3072);
+            const int64_t tiles = std::min<int64_t>(blocks, ((int64_t)INT32_MAX + 15) / 16), total = p.batch * tiles;
+            check(p.batch >= 1 && total + 65536 <= INT32_MAX, "tiles of a launch", total, p.batch, blocks);
+            for (int slices : {1, 384, 16384}) {
+                const int c = shared_chunk((int)total, slices, 128, (int)tiles, 64);
+                check(c >= 1 && (int64_t)c * slices >= total, "slices of a wide launch", c, slices, total);
+                const int d = slice_chunk(INT32_MAX, slices, 128, 4, (int)tiles, 64);
+                check(d >= 1 && (int64_t)d * slices >= INT32_MAX, "slices of the widest", d, slices);
+            }
+        }
     // slices of a plan: waves of a 256-CU GPU, the cap or a row per (sequence, 256 tokens)
     const size_t cap = kWsBytes;
     for (int nkv : {1, 2, 4, 8, 16})
