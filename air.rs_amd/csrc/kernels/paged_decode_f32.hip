@@ -16,8 +16,11 @@
 //   S = K . Q^T   lane (row r16 = lane % 16, g4 = lane / 16) holds 8 elements
 //                 of token r16 per 32 of head_dim (key_elem below); product
 //                 (m, e) contracts the four lanes' e-th ones.  bf16 pages
-//                 under bf16 queries take v_mfma_f32_16x16x32_bf16 instead,
-//                 whose operand is those 8 elements.  Where rows are whole
+//                 under bf16 queries, and 1-byte codes (exact in bf16) whose
+//                 scale holds for 32 elements, take v_mfma_f32_16x16x32_bf16
+//                 instead, whose operand is those 8 elements: f32 queries in
+//                 three bf16 parts (24 bits from 2^-110 on), the scale on each
+//                 32 elements' sum.  Where rows are whole
 //                 128-byte lines a load instruction reads eight of them, and a
 //                 transpose of one lane bit with the load index (DPP) gives
 //                 the lanes their elements; other rows are read directly, half
@@ -28,8 +31,8 @@
 //                 with head_dim dealt out in pieces of up to 16 bytes.
 // Every product is an f32 fused multiply-add (exact for bf16 operands); the
 // scores run in eight chains and a tile's P.V starts from zero, so the running
-// sums are rounded once per tile.  1-byte codes are dequantized (code * scale,
-// one rounding) in registers.
+// sums are rounded once per tile.  The values' 1-byte codes, and the keys' under
+// f32 products, are dequantized (code * scale, one rounding) in registers.
 //
 // The decode step's new token (k_new / v_new) is written to its page by the
 // wave that owns its sequence's last tile, just before it loads that tile:
@@ -40,7 +43,7 @@
 // pages.  48 sequences of 256 to 4096 tokens, 32 heads over 8: bf16 pages of 64
 // 49 us, 4.7 TB/s, 41 of them the slices' (180 us on the vector kernel this
 // replaced, four launches); f32 pages of 64 88 us, 5.2 TB/s (204); 64 sequences
-// of 256 to 8192 over int8 pages of 64 151 us, 2.3 TB/s (449).
+// of 256 to 8192 over int8 pages of 64 110 us, 3.2 TB/s (449).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -48,6 +51,7 @@
 
 #include "../host/status.hpp"
 #include "../pool.hpp"
+#include "bf16_parts.hpp"
 #include "codecs.hpp"
 #include "decode_common.hpp"
 #include "decode_slices.hpp"
@@ -190,20 +194,21 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // Waves per SIMD an instantiation is built for and launched with.
-template <int D, int PT, bool QB> constexpr int waves_per_simd() {
-    return PT == kF32 ? (D <= 64 ? 3 : 2)
-           : QB       ? (D <= 96 ? 4 : 3)
+template <int D, int PT, int QP> constexpr int waves_per_simd() {
+    return PT == kF32                  ? (D <= 64 ? 3 : 2)
+           : PT == kBf16 && QP == 1    ? (D <= 96 ? 4 : 3)
            : D <= 64  ? (PT == kBf16 ? 4 : 3)
            : D <= 96  ? 3
                       : (PT == kBf16 ? 3 : 2);
 }
 
-// D: a wave's columns.  QB: bf16 queries over bf16 pages (else the queries enter
-// as f32).  TEAM: the workgroup's waves share a slice, D columns of head_dim each.
-template <int D, int PT, bool QB, bool TEAM>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(waves_per_simd<D, PT, QB>(), waves_per_simd<D, PT, QB>())))
+// D: a wave's columns.  QP: the scores' products, 0 f32 (the queries as f32), 1 bf16
+// under bf16 queries, 3 bf16 under f32 queries in three parts.  TEAM: the
+// workgroup's waves share a slice, D columns of head_dim each.
+template <int D, int PT, int QP, bool TEAM>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(waves_per_simd<D, PT, QP>(), waves_per_simd<D, PT, QP>())))
 void decode_f32_kernel(DecodeArgs a) {
-    static_assert(!QB || PT == kBf16, "bf16 products take bf16 pages");
+    static_assert(QP == 0 || PT != kF32, "bf16 products take bf16 pages or codes");
     using P = Pieces<D, PT>;
     constexpr int EB = kElem<PT>, KM = D / 32;
     __shared__ int32_t s_pre[kMaxBatch + 2];
@@ -275,8 +280,8 @@ void decode_f32_kernel(DecodeArgs a) {
     auto key_elem = [&](int half) { return PT == kF32 ? 16 * half + 4 * g4 : 8 * g4 + 4 * half; };
     // ---- queries (head r16), the same elements; heads past the chunk and
     // columns past head_dim read zeros outside the descriptor
-    u32x4 qb[QB ? KM : 1];
-    float qf[QB ? 1 : KM][8];
+    u32x4 qb[QP ? QP : 1][QP ? KM : 1];
+    float qf[QP ? 1 : KM][8];
     auto load_q = [&](int bq) __attribute__((always_inline)) {
         const int qbytes = a.q_dtype == AIR_KV_F32 ? 4 : 2;
         const int64_t row = (int64_t)bq * a.n_q_heads + kh * G + g0;
@@ -284,8 +289,19 @@ void decode_f32_kernel(DecodeArgs a) {
 #pragma unroll
         for (int m = 0; m < KM; ++m) {
             const int off = (r16 * d + col0 + 32 * m) * qbytes;
-            if constexpr (QB) {
-                qb[m] = __builtin_amdgcn_raw_buffer_load_b128(rq, 32 * m < dw ? off + 16 * g4 : kOutside, 0, 0);
+            if constexpr (QP == 1) {
+                qb[0][m] = __builtin_amdgcn_raw_buffer_load_b128(rq, 32 * m < dw ? off + 16 * g4 : kOutside, 0, 0);
+            } else if constexpr (QP == 3) {
+                uint32_t x[8];
+                load_words<32, 0>(rq, 32 * m < dw ? off + 32 * g4 : kOutside, 0, x);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    uint32_t h, mid, l;
+                    split3(__uint_as_float(x[2 * j]), __uint_as_float(x[2 * j + 1]), h, mid, l);
+                    qb[0][m][j] = h;
+                    qb[1][m][j] = mid;
+                    qb[2][m][j] = l;
+                }
             } else {
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {
@@ -316,7 +332,7 @@ void decode_f32_kernel(DecodeArgs a) {
                                          : (r16 * d + 8 * g4) * EB);
     const int v_off = (4 * g4 * d + col0) * EB;
     uint32_t kw[KM][8 * EB / 4], vw[4][P::N][P::kMost * EB / 4 > 0 ? P::kMost * EB / 4 : 1];
-    float ksc[kByte<PT> ? KM : 1], vsc[kByte<PT> ? 4 : 1][kByte<PT> ? P::N : 1];
+    float ksc[kByte<PT> ? KM : 1][QP ? 4 : 1], vsc[kByte<PT> ? 4 : 1][kByte<PT> ? P::N : 1];
 
     __amdgpu_buffer_rsrc_t rv, rvs;
     auto load_values = [&]() __attribute__((always_inline)) {
@@ -391,10 +407,14 @@ void decode_f32_kernel(DecodeArgs a) {
         if constexpr (kByte<PT>) {
             const __amdgpu_buffer_rsrc_t rks = rsrc(a.k_scales + row0 * n_sc, nv * n_sc * 4);
             rvs = rsrc(a.v_scales + row0 * n_sc, nv * n_sc * 4);
+            // of the lane's own row, or (QP) of the four rows of its scores
 #pragma unroll
             for (int m = 0; m < KM; ++m)
-                ksc[m] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                    rks, 32 * m < dw ? (r16 * n_sc + ((col0 + 32 * m + 8 * g4) >> sg_log2)) * 4 : kOutside, 0, 0));
+#pragma unroll
+                for (int i = 0; i < (QP ? 4 : 1); ++i)
+                    ksc[m][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                        rks, 32 * m < dw ? ((QP ? 4 * g4 : r16) * n_sc + ((col0 + 32 * m + (QP ? 0 : 8 * g4)) >> sg_log2)) * 4 : kOutside,
+                        i * n_sc * 4, 0));
         }
         load_values();
         return ok;
@@ -470,13 +490,29 @@ void decode_f32_kernel(DecodeArgs a) {
         f32x4 part[KM];
 #pragma unroll
         for (int m = 0; m < KM; ++m) {
-            if constexpr (QB) {
-                part[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    __builtin_bit_cast(bf16x8, u32x4{kw[m][0], kw[m][1], kw[m][2], kw[m][3]}),
-                    __builtin_bit_cast(bf16x8, qb[m]), zero, 0, 0, 0);
+            if constexpr (QP) {
+                u32x4 ka;
+                if constexpr (PT == kBf16) {
+                    ka = u32x4{kw[m][0], kw[m][1], kw[m][2], kw[m][3]};
+                } else {
+                    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+                    float x[8];
+                    widen<PT, 8, FF>(kw[m], 1.0f, x);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        ka[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x[2 * j], x[2 * j + 1]}), bf16x2));
+                }
+                part[m] = zero;
+#pragma unroll
+                for (int p = QP - 1; p >= 0; --p)        // the least part first
+                    part[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        __builtin_bit_cast(bf16x8, ka), __builtin_bit_cast(bf16x8, qb[p][m]), part[m], 0, 0, 0);
+                if constexpr (kByte<PT>)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) part[m][i] *= ksc[m][QP ? i : 0];
             } else {
                 float x[8];
-                widen<PT, 8, FF>(kw[m], kByte<PT> ? ksc[m] : 1.0f, x);
+                widen<PT, 8, FF>(kw[m], kByte<PT> ? ksc[kByte<PT> ? m : 0][0] : 1.0f, x);
                 f32x4 c[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) c[e] = mfma4(x[e], qf[m][e], zero);
@@ -631,11 +667,11 @@ __global__ __launch_bounds__(kThreads) void decode_f32_merge_kernel(DecodeArgs a
     if (grp == 0 && mine) store_out<4>(a, oi, o);
 }
 
-template <int D, int PT, bool QB, bool TEAM>
+template <int D, int PT, int QP, bool TEAM>
 hipError_t launch_one(const DecodeArgs &a, hipStream_t s) {
     const int chunks = (a.group + kHeads - 1) / kHeads;
     const int64_t units = (int64_t)a.n_kv_heads * chunks * a.slices, per = TEAM ? 1 : kWaves;
-    hipLaunchKernelGGL((decode_f32_kernel<D, PT, QB, TEAM>), dim3((unsigned)((units + per - 1) / per)), dim3(kThreads),
+    hipLaunchKernelGGL((decode_f32_kernel<D, PT, QP, TEAM>), dim3((unsigned)((units + per - 1) / per)), dim3(kThreads),
                        0, s, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -648,10 +684,24 @@ hipError_t launch_one(const DecodeArgs &a, hipStream_t s) {
 
 template <int D, bool TEAM>
 hipError_t launch_d(const DecodeArgs &a, int dtype, hipStream_t s) {
-    if (dtype == AIR_KV_F32) return launch_one<D, kF32, false, TEAM>(a, s);
-    if (dtype == AIR_KV_INT8) return launch_one<D, kInt8, false, TEAM>(a, s);
-    if (dtype == AIR_KV_FP8) return launch_one<D, kFp8, false, TEAM>(a, s);
-    return a.q_dtype == AIR_KV_BF16 ? launch_one<D, kBf16, true, TEAM>(a, s) : launch_one<D, kBf16, false, TEAM>(a, s);
+    const bool q_bf16 = a.q_dtype == AIR_KV_BF16;
+    if (dtype == AIR_KV_F32) return launch_one<D, kF32, 0, TEAM>(a, s);
+    if (dtype == AIR_KV_BF16) return q_bf16 ? launch_one<D, kBf16, 1, TEAM>(a, s) : launch_one<D, kBf16, 0, TEAM>(a, s);
+    // Codes take f32 products where a scale holds for fewer than 32 elements, and
+    // fp8 codes past 64 columns under f32 queries (their two copies of a tile's
+    // arithmetic spill with three parts: 100 sequences of 400 to 800, 8 kv heads,
+    // pages of 96 70 us, 76 with them).  Elsewhere bf16 products are faster: 115
+    // of 4245 to 8491, 4 heads over 4, int8 pages of 64 130 us, 184 with f32
+    // products, 167 on the vector kernel before them.
+    const bool wide = a.scale_group >= 32;
+    if (dtype == AIR_KV_INT8)
+        return !wide    ? launch_one<D, kInt8, 0, TEAM>(a, s)
+               : q_bf16 ? launch_one<D, kInt8, 1, TEAM>(a, s)
+                        : launch_one<D, kInt8, 3, TEAM>(a, s);
+    if (wide && q_bf16) return launch_one<D, kFp8, 1, TEAM>(a, s);
+    if constexpr (D <= 64)
+        if (wide) return launch_one<D, kFp8, 3, TEAM>(a, s);
+    return launch_one<D, kFp8, 0, TEAM>(a, s);
 }
 
 // Past 128 elements a wave that holds a whole tile runs alone on its SIMD with
@@ -663,11 +713,11 @@ constexpr int kTeamColumns = 64;
 bool team(int d) { return d > 128; }
 
 template <int D> int waves_of(int dtype, bool q_bf16) {
-    return dtype == AIR_KV_F32    ? waves_per_simd<D, kF32, false>()
-           : dtype == AIR_KV_INT8 ? waves_per_simd<D, kInt8, false>()
-           : dtype == AIR_KV_FP8  ? waves_per_simd<D, kFp8, false>()
-           : q_bf16               ? waves_per_simd<D, kBf16, true>()
-                                  : waves_per_simd<D, kBf16, false>();
+    return dtype == AIR_KV_F32    ? waves_per_simd<D, kF32, 0>()
+           : dtype == AIR_KV_INT8 ? waves_per_simd<D, kInt8, 0>()
+           : dtype == AIR_KV_FP8  ? waves_per_simd<D, kFp8, 0>()
+           : q_bf16               ? waves_per_simd<D, kBf16, 1>()
+                                  : waves_per_simd<D, kBf16, 0>();
 }
 
 }  // namespace

@@ -101,8 +101,8 @@ def test_decode_f32_one_partition(dtype, d):
     assert torch.equal(out, one) and bool(torch.isfinite(out).all())
 
 
-@pytest.mark.parametrize("d", [64, 96])
-def test_decode_f32_every_fp8_code(d):
+@pytest.mark.parametrize("d,q_bf16", [(64, False), (96, False), (64, True), (96, True)])
+def test_decode_f32_every_fp8_code(d, q_bf16):
     """Pages written as raw blocks may hold any code: subnormal ones, which the
     format reads as zero, and 0xFF, which it reads as -480 (0x7F, NaN, is left
     out), here in single tiles of a sequence; and an entry outside the pool is
@@ -124,15 +124,17 @@ def test_decode_f32_every_fp8_code(d):
            for x in (host.k, host.v, host.k_scales, host.v_scales)]
     pool.write_blocks(np.arange(pool.num_blocks, dtype=np.int32), np.concatenate(raw, 1))
     lens = np.array([n], np.int32)
-    q = rng.standard_normal((1, kv * group, d)).astype(np.float32)
+    qt = torch.from_numpy(rng.standard_normal((1, kv * group, d)).astype(np.float32)).cuda()
+    qt = qt.to(torch.bfloat16) if q_bf16 else qt
+    q = qt.float().cpu().numpy()
     out = torch.empty(q.shape, device="cuda")
-    pool.paged_decode(torch.from_numpy(q).cuda(), torch.from_numpy(tables).cuda(), torch.from_numpy(lens).cuda(), out)
+    pool.paged_decode(qt, torch.from_numpy(tables).cuda(), torch.from_numpy(lens).cuda(), out)
     want = host.paged_decode(q, tables, lens, chunk=64)
     assert np.isfinite(want).all() and rel_err(out.cpu().numpy(), want) <= TOL_F32
     # the last block's entry outside the pool: as if the sequence ended before it
     assert pool.error_count(reset=True) == 0
     tables[0, n // bs] = pool.num_blocks + 3
-    pool.paged_decode(torch.from_numpy(q).cuda(), torch.from_numpy(tables).cuda(), torch.from_numpy(lens).cuda(), out)
+    pool.paged_decode(qt, torch.from_numpy(tables).cuda(), torch.from_numpy(lens).cuda(), out)
     want = host.paged_decode(q, tables, np.array([n // bs * bs], np.int32), chunk=64)
     assert rel_err(out.cpu().numpy(), want) <= TOL_F32
     assert pool.error_count(reset=True) > 0
