@@ -196,7 +196,7 @@ __device__ __forceinline__ void lds_barrier() {
 // Waves per SIMD an instantiation is built for and launched with.
 template <int D, int PT, int QP> constexpr int waves_per_simd() {
     return PT == kF32                  ? (D <= 64 ? 3 : 2)
-           : PT == kBf16 && QP == 1    ? (D <= 96 ? 4 : 3)
+           : PT == kBf16 && QP == 1    ? (D <= 96 ? 4 : D <= 128 ? 3 : 2)
            : D <= 64  ? (PT == kBf16 ? 4 : 3)
            : D <= 96  ? 3
                       : (PT == kBf16 ? 3 : 2);
@@ -676,7 +676,7 @@ hipError_t launch_one(const DecodeArgs &a, hipStream_t s) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const dim3 grid((unsigned)a.batch, (unsigned)a.n_kv_heads, (unsigned)((a.group + kWaves - 1) / kWaves));
-    if constexpr (TEAM) hipLaunchKernelGGL(decode_f32_merge_kernel<256>, grid, dim3(kThreads), 0, s, a);
+    if constexpr (TEAM || D > 128) hipLaunchKernelGGL(decode_f32_merge_kernel<256>, grid, dim3(kThreads), 0, s, a);
     else if constexpr (D <= 64) hipLaunchKernelGGL(decode_f32_merge_kernel<64>, grid, dim3(kThreads), 0, s, a);
     else hipLaunchKernelGGL(decode_f32_merge_kernel<128>, grid, dim3(kThreads), 0, s, a);
     return hipGetLastError();
@@ -712,6 +712,17 @@ hipError_t launch_d(const DecodeArgs &a, int dtype, hipStream_t s) {
 constexpr int kTeamColumns = 64;
 bool team(int d) { return d > 128; }
 
+// Two waves of bf16 products fit a SIMD with a whole tile each, and need no
+// barrier: under bf16 queries a launch over bf16 pages takes them where they have
+// 20 tiles a SIMD to walk and the partitions alone are as many (16 sequences of
+// 6000 to 12000, 16 heads over 8, pages of 160: 148 us, 188 shared by four; 5 of 2459
+// to 19678, 16 over 4, pages of 256, below both: 70 and 46).  The table's width
+// stands for the lengths.
+bool lone_bf16(const air_kv_pool &p, int64_t per_slice, int64_t batch, int64_t tiles, int64_t max_splits) {
+    return team(p.desc.head_dim) && p.desc.dtype == AIR_KV_BF16 && batch * tiles * per_slice >= (int64_t)80 * p.cus &&
+           batch * std::min(tiles, max_splits) * per_slice >= (int64_t)8 * p.cus;
+}
+
 template <int D> int waves_of(int dtype, bool q_bf16) {
     return dtype == AIR_KV_F32    ? waves_per_simd<D, kF32, 0>()
            : dtype == AIR_KV_INT8 ? waves_per_simd<D, kInt8, 0>()
@@ -728,7 +739,10 @@ int plan_decode_f32(const air_kv_pool &p, int32_t n_q_heads, int32_t batch, int3
                     int32_t max_splits, DecodePlan *plan) {
     const int nkv = p.desc.n_kv_heads, d = p.desc.head_dim, dt = p.desc.dtype;
     const int64_t per_slice = (int64_t)nkv * ((n_q_heads / nkv + kHeads - 1) / kHeads);
+    const int64_t tiles = std::min<int64_t>(((int64_t)max_blocks * p.desc.block_size + 15) / 16, INT32_MAX);
+    plan->lone = lone_bf16(p, per_slice, batch, tiles, max_splits);
     auto waves = [&](bool q_bf16) {
+        if (q_bf16 && plan->lone) return (int64_t)p.cus * 4 * waves_per_simd<256, kBf16, 1>();
         const int wps = d <= 64    ? waves_of<64>(dt, q_bf16)
                         : d <= 96  ? waves_of<96>(dt, q_bf16)
                         : !team(d) ? waves_of<128>(dt, q_bf16)
@@ -756,7 +770,8 @@ hipError_t launch_decode_f32(const DecodeArgs &base, const DecodePlan &plan, voi
         a.batch = std::min(base.batch - b0, plan.batch_per_launch);
         a.slices = base.q_dtype == AIR_KV_F32 ? plan.slices_qf32 : plan.slices;
         a.slots = plan.slots;
-        a.simd_slices = team(d) ? (base.simd_slices + kWaves - 1) / kWaves : base.simd_slices;
+        const bool lone = plan.lone && base.q_dtype == AIR_KV_BF16;
+        a.simd_slices = team(d) && !lone ? (base.simd_slices + kWaves - 1) / kWaves : base.simd_slices;
         const int64_t q_row = (int64_t)b0 * a.n_q_heads * d;
         a.q = (const char *)base.q + q_row * (base.q_dtype == AIR_KV_F32 ? 4 : 2);
         a.out = (char *)base.out + q_row * (base.out_dtype == AIR_KV_F32 ? 4 : 2);
@@ -777,6 +792,7 @@ hipError_t launch_decode_f32(const DecodeArgs &base, const DecodePlan &plan, voi
         const hipError_t e = d <= 64    ? launch_d<64, false>(a, plan.dtype, s)
                              : d <= 96  ? launch_d<96, false>(a, plan.dtype, s)
                              : !team(d) ? launch_d<128, false>(a, plan.dtype, s)
+                             : lone     ? launch_one<256, kBf16, 1, false>(a, s)
                                         : launch_d<kTeamColumns, true>(a, plan.dtype, s);
         if (e != hipSuccess) return e;
     }

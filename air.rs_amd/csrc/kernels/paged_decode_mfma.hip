@@ -1034,6 +1034,7 @@ int plan_decode_mfma(const air_kv_pool &p, int32_t n_q_heads, int32_t batch, int
     };
     const int64_t slices = slices_for(waves_per_simd(p.desc.dtype));
     plan->mfma = true;
+    plan->lone = false;
     plan->seq_pieces = 0;
     plan->dtype = p.desc.dtype;
     plan->slices = (int32_t)slices;

@@ -41,6 +41,7 @@ struct DecodePlan {
     int32_t slices_append;  // the same for the fused append + decode
     int32_t batch_per_launch;
     int32_t max_splits;   // partitions of a sequence at most
+    bool lone;            // paged_decode_f32.hip past head_dim 128: a wave to a tile under bf16 queries
     int32_t seq_pieces;   // slices of each sequence's own (0: of the batch's tiles)
     int32_t slots;        // partial rows per (kv head, q head of the group)
     size_t ws_bytes;

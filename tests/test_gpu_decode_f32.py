@@ -85,6 +85,29 @@ def test_decode_f32_wide_batches(dtype, d, n_kv, group, batch, bad):
     assert pa.error_count() > 0 and pb.error_count() > 0
 
 
+@pytest.mark.parametrize("d,n_kv,group,batch,width", [(256, 4, 4, 40, 130), (160, 8, 2, 300, 24), (224, 2, 20, 70, 160)])
+def test_decode_f32_wide_heads_lone_waves(d, n_kv, group, batch, width):
+    """bf16 queries over bf16 pages past 128 elements where the launch is wide
+    enough (by its table) for a wave to a tile: the step's pages and outputs, and
+    few splits."""
+    ctx = [(37 * i) % 300 for i in range(batch)]
+    cfg = workloads.Config("lone", n_kv * group, n_kv, d, 16, airkv.BF16, batch)
+    w, pa, pb, host, tables, lens, k_new, v_new = _setup(cfg, ctx, seed=51 + d)
+    tables = np.pad(tables, ((0, 0), (0, max(0, width - tables.shape[1]))), constant_values=-1)
+    q = np.random.default_rng(11).standard_normal((batch, n_kv * group, d)).astype(np.float32)
+    q, got = _run_pair(cfg, pa, pb, host, tables, lens, k_new, v_new, q, q_f32=False)
+    want = host.paged_decode(q, tables, lens, chunk=64)
+    err = rel_err(got, want)
+    torch = torch_mod()
+    qt, tt, lt = torch.from_numpy(q).cuda().to(torch.bfloat16), torch.from_numpy(tables).cuda(), torch.from_numpy(lens).cuda()
+    for most in (1, 8):
+        out = torch.full(q.shape, float("nan"), device="cuda")
+        pb.paged_decode(qt, tt, lt, out, max_splits=most)
+        err = max(err, rel_err(out.cpu().numpy(), want))
+    log(f"decode f32 lone waves d={d}: rel err {err:.2e}")
+    assert err <= TOL_F32
+
+
 @pytest.mark.parametrize("dtype,d", [(airkv.BF16, 64), (airkv.INT8, 96), (airkv.F32, 224)])
 def test_decode_f32_one_partition(dtype, d):
     """max_splits 1: a sequence's result does not depend on the others of its
